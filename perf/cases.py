@@ -74,7 +74,7 @@ def draw(rng):
         op = rng.choice(["matmul", "matmul", "matmul", "ffn", "moe"])
         if op == "matmul":
             w = rng.choice(types)
-            k = 32 * _log(rng, 16, 576) if w == "q8_0" else 256 * _log(rng, 2, 72)
+            k = 64 * _log(rng, 8, 288) if w == "q8_0" else 256 * _log(rng, 2, 72)
             c = dict(op=op, w=w, m=_log(rng, 1, 2048), n=_log(rng, 512, 152064), k=k,
                      x=rng.choice(["f32", "f32", "f16"]))
         elif op == "ffn":
