@@ -30,28 +30,28 @@ ACTS = {"silu": None, "gelu": arf_amd.arfq.ACT_GELU_TANH}
 def listed():
     return [
         # one projection of a small model, one token: launch and latency
-        dict(name="q8_0 decode, small", op="matmul", w="q8_0", m=1, n=2048, k=2048, x="f32"),
+        dict(name="q8_0 decode small", op="matmul", w="q8_0", m=1, n=2048, k=2048, x="f32"),
         # gate or up projection of a dense model, one token
         dict(name="q4_k decode", op="matmul", w="q4_k", m=1, n=17408, k=5120, x="f32"),
         # the vocabulary projection, one token: the largest matrix of a model
-        dict(name="q6_k head, decode", op="matmul", w="q6_k", m=1, n=151936, k=5120, x="f32"),
+        dict(name="q6_k head decode", op="matmul", w="q6_k", m=1, n=151936, k=5120, x="f32"),
         # the FFN of one decode step, in the usual mix of formats (down in Q6_K)
-        dict(name="ffn decode, q4_k/q6_k", op="ffn", w="q4_k", down="q6_k", m=1, hidden=5120, inter=17408, act="silu"),
+        dict(name="ffn decode q4_k+q6_k", op="ffn", w="q4_k", down="q6_k", m=1, hidden=5120, inter=17408, act="silu"),
         # down projection for eight sequences, or eight drafted tokens
         dict(name="q6_k batch 8", op="matmul", w="q6_k", m=8, n=5120, k=17408, x="f32"),
         # gate projection for a ragged batch of sequences
         dict(name="q5_k batch 45", op="matmul", w="q5_k", m=45, n=17408, k=5120, x="f32"),
         # prompt of 2048 tokens, activations kept in f16
-        dict(name="q4_k prefill 2048, f16", op="matmul", w="q4_k", m=2048, n=17408, k=5120, x="f16"),
+        dict(name="q4_k prefill 2048 f16", op="matmul", w="q4_k", m=2048, n=17408, k=5120, x="f16"),
         # a projection over a prompt of odd length, f32 activations
         dict(name="iq4_xs prefill 777", op="matmul", w="iq4_xs", m=777, n=4100, k=5120, x="f32"),
         # the FFN over a short prompt, f32 activations, the other gate activation
-        dict(name="ffn prefill 333, gelu", op="ffn", w="q4_k", down="q6_k", m=333, hidden=4096, inter=11008, act="gelu"),
+        dict(name="ffn prefill 333 gelu", op="ffn", w="q4_k", down="q6_k", m=333, hidden=4096, inter=11008, act="gelu"),
         # the MoE block for four sequences decoding
         dict(name="moe decode 4", op="moe", w="q4_k", down="q4_k", experts=128, topk=8, tokens=4, hidden=2048,
              inter=768, x="f32"),
         # the MoE block for a ragged batch, the usual mix of formats
-        dict(name="moe batch 37, q4_k/q6_k", op="moe", w="q4_k", down="q6_k", experts=128, topk=8, tokens=37,
+        dict(name="moe batch 37 q4_k+q6_k", op="moe", w="q4_k", down="q6_k", experts=128, topk=8, tokens=37,
              hidden=2048, inter=768, x="f32"),
         # the MoE block over a prompt of 512 tokens
         dict(name="moe prefill 512", op="moe", w="q4_k", down="q4_k", experts=128, topk=8, tokens=512, hidden=2048,
