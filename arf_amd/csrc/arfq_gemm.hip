@@ -336,26 +336,24 @@ static int64_t bd_stream_bytes(int qtype) {
 
 static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-GemmPlan gemm_plan(const arfq_weight *w, int64_t m, int x_dtype, bool x16) {
+// direct: the direct-operand kernel where it takes the product
+static GemmPlan gemm_plan_of(const arfq_weight *w, int64_t m, int x_dtype, bool x16, bool direct) {
     GemmPlan p;
     const int cus = w->ctx && w->ctx->cus > 0 ? w->ctx->cus : 256;
     const bool kind2 = w->qtype == ARFQ_Q4_K || w->qtype == ARFQ_Q5_K;  // min term: x sums
     p.skinny = m <= 64 && w->k % 256 == 0;
     p.bm = m > 64 ? 128 : 64;
-    // prefill: the direct-operand kernel (one launch, no split-K) for every
-    // format but IQ4_XS at f32 x (its weights are rounded to f16, so its x
-    // keeps the hi + lo split of the tile loop below)
+    // prefill: the direct-operand kernel (one launch, no split-K)
     const int64_t bdb = bd_stream_bytes(w->qtype);
     // (an f32 x enters it as hi + lo rows unless x16: twice the x bytes)
     const int64_t bdx = x_dtype == ARFQ_F32 && !x16 ? 2 : 1;
-    p.bd = !p.skinny && m > 64 && bdb && w->k % 256 == 0 && !(w->qtype == ARFQ_IQ4_XS && x_dtype == ARFQ_F32) &&
-           w->n * (w->k / 256) * bdb < ((int64_t)1 << 31) && bdx * m * w->k * 2 < ((int64_t)1 << 31);  // buffer loads
+    p.bd = direct && !p.skinny && m > 64 && bdb && w->k % 256 == 0 && w->n * (w->k / 256) * bdb < ((int64_t)1 << 31) && bdx * m * w->k * 2 < ((int64_t)1 << 31);  // buffer loads
     // f32 x: scaled per row by a power of two into f16 range, then split into
     // f16 parts for the skinny kernel and the direct-operand prefill (hi + lo
     // rows: its tiles cover 64 rows at twice the MFMAs; one f16 part under x16),
-    // or into f16 hi + lo for the tile loop (IQ4_XS prefill, whose weights are
-    // rounded to f16: this way only one of the two operands is); the output
-    // rows are multiplied back by the scale
+    // or into f16 hi + lo for the tile loop (whose weights are rounded to f16:
+    // this way only one of the two operands is); the output rows are multiplied
+    // back by the scale
     p.xsplit = !p.skinny && !p.bd && x_dtype == ARFQ_F32;
     p.convert = x_dtype == ARFQ_F32;
     // skinny kernel, f32 x: m <= 8 as three f16 parts (one 32-row x tile holds
@@ -428,6 +426,18 @@ GemmPlan gemm_plan(const arfq_weight *w, int64_t m, int x_dtype, bool x16) {
     else
         o += p.splits > 1 ? al256((size_t)p.splits * m * w->n * 4) : al256(bd_part);
     p.scratch_bytes = o;
+    return p;
+}
+
+GemmPlan gemm_plan(const arfq_weight *w, int64_t m, int x_dtype, bool x16, size_t limit) {
+    const GemmPlan p = gemm_plan_of(w, m, x_dtype, x16, true);
+    // IQ4_XS at f32 x: which products a caller's scratch is enough for goes by the
+    // tile loop's need, and one that the direct kernel's partials do not fit in
+    // runs the tile loop
+    if (limit != SIZE_MAX && p.bd && w->qtype == ARFQ_IQ4_XS && x_dtype == ARFQ_F32) {
+        const GemmPlan t = gemm_plan_of(w, m, x_dtype, x16, false);
+        if (t.scratch_bytes > limit || p.scratch_bytes > limit) return t;
+    }
     return p;
 }
 

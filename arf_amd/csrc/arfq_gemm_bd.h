@@ -289,12 +289,15 @@ struct BdQ5K {
     }
 };
 
-// IQ4_XS (weights rounded to f16): step p, lane half h = sub-block 2p + h,
-// whose 16 code bytes hold elements 0..15 in the low nibbles and 16..31 in the
-// high ones; group kk = elements 8kk .. 8kk + 7 (nibble kk / 2 of bytes
-// 8 (kk % 2) .. + 7).  Operands (ls - 32) * kv in units of d, rounded once to
-// f16 (exact while |(ls - 32) kv| <= 2048); kv from the codebook with two
-// v_perm.  (dequant_iq4_xs, crates/arf-core/src/model/gguf.rs:1937-1976)
+// IQ4_XS: step p, lane half h = sub-block 2p + h, whose 16 code bytes hold
+// elements 0..15 in the low nibbles and 16..31 in the high ones; group kk =
+// elements 8kk .. 8kk + 7 (nibble kk / 2 of bytes 8 (kk % 2) .. + 7).  Operands
+// (ls - 32) * kv in units of d, rounded once to f16 (exact while |(ls - 32) kv|
+// <= 2048); kv from the codebook with two v_perm.  f32 x enters as hi + lo rows
+// here too: 149.5 -> 98.0 us at 777 x 5120 -> 4100 against the tile loop, which
+// dequantizes into LDS and reads both operands of every MFMA from there (error
+// against 64 bits 2.1e-4 -> 1.7e-4: the tile loop rounds every weight).
+// (dequant_iq4_xs, crates/arf-core/src/model/gguf.rs:1937-1976)
 struct BdIQ4XS {
     static constexpr int XPARTS = 2;
     static constexpr bool EXTRA = false;

@@ -393,7 +393,7 @@ int arfq_matmul_noalloc(arfq_ctx *ctx, const arfq_weight *w, int expert, int64_t
         // the decode GEMVs use no scratch
         e = arfq::launch_gemv(w, expert, m, (const float *)x, y, ctx->stream, x16);
     } else if (arfq::gemm_supports(w, m)) {
-        const arfq::GemmPlan plan = arfq::gemm_plan(w, m, x_dtype, x16);
+        const arfq::GemmPlan plan = arfq::gemm_plan(w, m, x_dtype, x16, ARFQ_NOALLOC_SCRATCH_BYTES);
         if (plan.scratch_bytes > ARFQ_NOALLOC_SCRATCH_BYTES)
             return fail(ctx, ARFQ_E_UNSUPPORTED,
                         "matmul_noalloc: this product needs " + std::to_string(plan.scratch_bytes) +

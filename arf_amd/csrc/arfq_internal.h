@@ -142,7 +142,8 @@ struct GemmPlan {
     size_t off_xh = 0, off_xl = 0, off_xs = 0, off_rs = 0, off_part = 0, scratch_bytes = 0;
 };
 // x16: ARFQ_OPT_GEMV_X16 is set (the skinny and prefill kernels take an f32 x as one f16 part)
-GemmPlan gemm_plan(const arfq_weight *w, int64_t m, int x_dtype, bool x16 = false);
+// limit: the scratch a caller with a fixed one has; a plan above it does not run there
+GemmPlan gemm_plan(const arfq_weight *w, int64_t m, int x_dtype, bool x16 = false, size_t limit = SIZE_MAX);
 bool gemm_supports(const arfq_weight *w, int64_t m);
 // y[m, n] = x[m, k] . W_e^T; `scratch` holds plan.scratch_bytes.
 hipError_t launch_gemm(const arfq_weight *w, int e, int64_t m, const void *x, int x_dtype,

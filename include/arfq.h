@@ -142,8 +142,8 @@ int arfq_weight_info(const arfq_weight *w, int *qtype, int64_t *n_rows, int64_t 
  * and Q8_0 (Q6_K scales beyond +-64 and Q8_0's d * q as two f16 operands
  * above 64 rows), except in the tile loop that takes the shapes the direct
  * prefill kernel does not (Q8_0 with k not a multiple of 256, streams past
- * 2 GiB) and IQ4_XS above 64 rows at f32 x: there the dequant is rounded once
- * to f16.
+ * 2 GiB): there the dequant is rounded once to f16.  IQ4_XS weights are exact
+ * up to 64 rows; above, (ls - 32) * kv is rounded to f16 where it passes 2048.
  * Replaces add_matmul_m / add_matmul
  * (crates/arf-gpu/src/gpu/dispatch.rs:169-202, Q4KS arms :517-630) and the
  * island's gemv_q4ks / gemv_q4ks_batch / matmul_mm_q4ks selection
