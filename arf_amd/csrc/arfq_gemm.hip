@@ -362,7 +362,9 @@ static GemmPlan gemm_plan_of(const arfq_weight *w, int64_t m, int x_dtype, bool 
     // half of the 32-row tile at m <= 16 (no extra MFMAs), a second tile at
     // m <= 32 and two more at m <= 64 (twice the MFMAs).  With x16
     // (ARFQ_OPT_GEMV_X16): one part, x rounded to f16.
-    p.parts = p.skinny && x_dtype == ARFQ_F32 && !x16 ? (m <= 8 ? 3 : 2) : p.bd && bdx == 2 ? 2 : 1;
+    // Q6_K and Q8_0 at m <= 4 have no 16-bit form to opt into and stay exact.
+    const bool exact4 = m <= 4 && (w->qtype == ARFQ_Q6_K || w->qtype == ARFQ_Q8_0);
+    p.parts = p.skinny && x_dtype == ARFQ_F32 && (!x16 || exact4) ? (m <= 8 ? 3 : 2) : p.bd && bdx == 2 ? 2 : 1;
     // three parts (and their sub-block sums): formed by the skinny kernel as it
     // stages x (no preparation launch, no scratch for x)
     p.fx = p.skinny && p.parts == 3;
@@ -445,7 +447,7 @@ template <class F, int TA, int PARTS, int GM = 0xFF, class XT = _Float16>
 static hipError_t launch_sk_t(const F &fmt, const arfq_weight *w, int64_t m, const XT *x,
                               const uint16_t *xs, const float *rs, int rss, float *y, float *part,
                               int S, hipStream_t s) {
-    if constexpr (F::KIND == 4 && TA == 1 && GM == 0xFF) {
+    if constexpr (F::KIND >= 3 && TA == 1 && GM == 0xFF) {
         // at most 8 rows (8 hi + 8 lo with two parts, + 8 mid with three): the
         // per-sub-block scaling touches only the accumulator groups that hold them
         if (m <= 8)

@@ -10,7 +10,8 @@
 //     codes); m = 2..4 and ARFQ_OPT_GEMV_X16: gemv_dot<Fmt> (x in 16-bit fixed
 //     point, integer dots); the same step walk; gemv_q6k is the fallback for
 //     shapes neither takes.
-//   * Q8_0: gemv_q80w, one wave per row, f32.
+//   * Q8_0: gemv_q80w, one wave per two rows, f32.
+//   Large Q6_K and Q8_0 products at m = 2..4 go to the skinny MFMA kernel.
 // Reference behaviour: matmul_vec_q4ks_msl.metal:46-165 (simdgroup strides
 // sub-blocks, s*sum(q*x) + lo*sum(x) per sub-block, simd_sum), and the oracle
 // dot_q4ks (crates/arf-ml/src/matmul.rs:327-358), matmul_nt_q8_0 (:174-204).
@@ -1751,13 +1752,30 @@ static bool q4k_x16_ok(const arfq_weight *w, int64_t m) {
            w->n * (w->k / 256) * 128 < (int64_t)Q4K_OOB;
 }
 
+// Q6_K and Q8_0 at m = 2..4: where the skinny MFMA kernel (x as three f16 parts,
+// exact products) is faster than the GEMVs, whose lanes read x again for every
+// weight row.  Its launch and the split-K add cost ~9.5 us at any size, so the
+// line lies where the GEMV passes that.  Q6_K's GEMV walks k in turns of 2048
+// and loses from k = 4096 on at any n (m = 2, 300 x 16384: 29.9 -> 13.1 us; 2048
+// x 4096: 10.0 -> 9.7), below that with the work (m = 4, 20000 x 2048: 28.8 ->
+// 18.7; 2048 x 2048: 8.2 against 9.6).  Q8_0 from ~30M products on (m = 4,
+// 4096 x 4096: 19.1 -> 10.3; m = 3, 17408 -> 5120: 73 -> 26; m = 3, 4096 x 2048:
+// 8.5 against 9.9), not for the few rows that leave its waves short (1000 x
+// 18432: 14.6 against 15.6).  Error against 64 bits: 1.7e-7 -> 1.2e-7 (Q6_K),
+// unchanged at 1e-7 (Q8_0).
+static bool skinny_m2_4(const arfq_weight *w, int64_t m) {
+    if (m < 2 || w->k % 256 != 0 || w->n > INT32_MAX / 2 || w->k > INT32_MAX / 2) return false;
+    const bool much = w->n * w->k >= 30000000 / m;
+    return w->qtype == ARFQ_Q6_K ? w->k >= 4096 || much : much && w->n >= 1024;
+}
+
 // Which (qtype, m) the GEMV family takes.  Without x16 every path multiplies
 // f32 x in f32: Q4_K / Q5_K / IQ4_XS / Q6_K at m = 1 (the exact-code f32
-// kernels, while their LDS fits), Q6_K at m = 2..4 (gemv_q6k) and Q8_0 at
-// m <= 4 (gemv_q80w).  Q4_K / Q5_K / IQ4_XS at m = 2..4, and m = 1 shapes too
-// long for the f32 kernels' LDS, go to the skinny MFMA GEMM (x as f16 hi + lo).
-// With x16 the 16-bit kernels take the shapes they fit; the rest keep the
-// f32 path.
+// kernels, while their LDS fits), small Q6_K products at m = 2..4 (gemv_q6k) and
+// small Q8_0 ones at m <= 4 (gemv_q80w).  Q4_K / Q5_K / IQ4_XS at m = 2..4, and
+// m = 1 shapes too long for the f32 kernels' LDS, go to the skinny MFMA GEMM (x
+// as three f16 parts).  With x16 the 16-bit kernels take the shapes they fit;
+// the rest keep the f32 path.
 bool gemv_supports(const arfq_weight *w, int64_t m, bool x16) {
     if (m < 1 || m > GEMV_MAX_M) return false;
     switch (w->qtype) {
@@ -1769,8 +1787,9 @@ bool gemv_supports(const arfq_weight *w, int64_t m, bool x16) {
         if (x16 && dot_ok(w, m)) return true;
         return m == 1 && dot_f32_ok(w);
     case ARFQ_Q6_K:  // gemv_q6k takes what the dot kernels do not
+        return (x16 && dot_ok(w, m)) || !skinny_m2_4(w, m);
     case ARFQ_Q8_0:
-        return true;
+        return !skinny_m2_4(w, m);
     default:
         return false;
     }

@@ -64,6 +64,7 @@ __device__ __forceinline__ half8 u4_to_h8(uint32_t a, uint32_t b, uint32_t c, ui
 // the lane's sub-block (elements 8kk .. 8kk + 7, sigma nibble order).
 struct SkQ4K {
     static constexpr int KIND = 2, RB = 128;
+    static constexpr bool OWN = false;
     struct Blk {
         u32x4 h;
     };
@@ -129,6 +130,7 @@ struct SkQ6K {
     // 16-element sub-block, whose product is scaled by its own d * sc in f32
     // (KIND 4)
     static constexpr int KIND = 4, RB = 192;
+    static constexpr bool OWN = false;
     struct Blk {
         u32x4 sc;  // the 16 i8 scales
         uint32_t d;
@@ -203,6 +205,7 @@ struct SkQ6K {
 // |sc| <= 62 (33 * 63 needs 12 bits).  Same slab layout and step map as SkQ6K.
 struct SkQ6KI : SkQ6K {
     static constexpr int KIND = 1;
+    static constexpr bool OWN = false;
     __host__ __device__ SkQ6KI shifted(int64_t nb) const { return {SkQ6K::shifted(nb)}; }
     __device__ static float2 scale(const Blk &k) { return make_float2(2.f * h2f(k.d), 0.f); }
     __device__ static void frag(const uint8_t *srow, const Blk &k, int p, int h, half8 f[4]) {
@@ -241,6 +244,7 @@ struct SkQ80 {
     // block 2p, MFMAs 2, 3 block 2p + 1, and each block's product is scaled by
     // its own d in f32 (KIND 3, as IQ4_XS)
     static constexpr int KIND = 3, RB = 256;
+    static constexpr bool OWN = true;
     struct Blk {
         u32x4 d;  // the 8 f16 scales of the 8 Q8_0 blocks
     };
@@ -291,6 +295,7 @@ struct SkQ80 {
 // (dequant_q5_k, crates/arf-core/src/model/gguf.rs:2053-2090)
 struct SkQ5K {
     static constexpr int KIND = 2, RB = 160;
+    static constexpr bool OWN = false;
     using Blk = SkQ4K::Blk;
     const uint4 *hdr;
     const uint8_t *q;
@@ -340,6 +345,7 @@ struct SkQ5K {
 // (dequant_iq4_xs, crates/arf-core/src/model/gguf.rs:1937-1976)
 struct SkIQ4XS {
     static constexpr int KIND = 3, RB = 128;
+    static constexpr bool OWN = false;
     struct Blk {
         u32x2 h;  // d | scales_h << 16, scales_l
     };
@@ -427,15 +433,20 @@ constexpr size_t sk_lds() {
 // F::a_off) and, for KIND 2, whose sub-block sums (bf16 hi[8] | lo[8]) start
 // at srow(t); then the block end of KIND 1 / 2 (the min term's two MFMAs
 // into acc, then acc += d * cb).  cb and cq are the block's own accumulators.
-// (GM, MERGE, PIN:
-// as skinny_loop.)
-template <class F, int TA, int TU, int NW, int GM, bool MERGE, bool PIN, class XRow, class SRow>
+// (GM, MERGE, PIN: as skinny_loop.)  OWN (KIND 3): the block's sub-blocks are
+// summed apart and then added to acc, so a long K range is a sum of block sums
+// instead of one chain of 8 terms per block (Q8_0 at m = 2, k = 5120: error
+// against 64 bits 1.5e-7 -> 9.4e-8, the f32 GEMV's 9.8e-8; IQ4_XS, which has no
+// GEMV at m > 1 to match, ran 6 % longer with it).
+template <class F, int TA, int TU, int NW, int GM, bool MERGE, bool PIN, bool OWN = false, class XRow, class SRow>
 __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::Blk (&wbk)[NW], XRow xrow,
                                          SRow srow, int lr, int h, floatx16 (&acc)[NW][TA], floatx16 (&cb)[NW][TA],
                                          floatx16 (&cq)[NW][F::KIND == 3 ? TA : 1]) {
     constexpr int KIND = F::KIND;
     constexpr int TO = MERGE ? TU / 2 : TU;  // accumulator tiles written
     constexpr int SL = F::RB + 16;           // slab row stride (bytes)
+    static_assert(!OWN || KIND == 3, "block sums apart: scaled per sub-block");
+    floatx16 own[OWN ? NW : 1][OWN ? TO : 1];
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         if constexpr (PIN && TO == 2) __builtin_amdgcn_sched_barrier(0);
@@ -491,8 +502,16 @@ __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::
 #pragma unroll
                 for (int ti = 0; ti < TO; ti++)
 #pragma unroll
-                    for (int i = 0; i < 16; i++)
-                        acc[w][ti][i] = fmaf(ss.y, cq[w][ti][i], fmaf(ss.x, cb[w][ti][i], acc[w][ti][i]));
+                    for (int i = 0; i < 16; i++) {
+                        if (!((GM >> (4 * ti + (i >> 2))) & 1)) continue;
+                        if constexpr (OWN) {
+                            const float v = p == 0 ? ss.x * cb[w][ti][i] : fmaf(ss.x, cb[w][ti][i], own[w][ti][i]);
+                            own[w][ti][i] = fmaf(ss.y, cq[w][ti][i], v);
+                            if (p == 3) acc[w][ti][i] += own[w][ti][i];
+                        } else {
+                            acc[w][ti][i] = fmaf(ss.y, cq[w][ti][i], fmaf(ss.x, cb[w][ti][i], acc[w][ti][i]));
+                        }
+                    }
             }
         }
     }
@@ -529,7 +548,7 @@ __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::
 // wrow0[w] + 31 (rows past nrows are clamped: computed, never to be stored).
 // The block loop of skinny_run for the first TU (<= TA) x tiles.
 // GM: the 8-row accumulator groups (bit 4 t + g: rows 32 t + 8 g .. + 7) that
-// hold real rows; KIND 4 scales only those (the others stay 0).  MERGE: the
+// hold real rows; KIND 3 and 4 scale only those (the others stay 0).  MERGE: the
 // second half of the x tiles (TU / 2 .. TU - 1) holds the low halves of the
 // first half's rows (f32 x as f16 hi + lo), so tile t's products go into tile
 // t % (TU / 2)'s accumulators (the second half of acc is left as it is).  PIN:
@@ -730,7 +749,7 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
         // keep the scheduler from sinking the loads: they must be in flight
         // during this block, not issued at its end
         __builtin_amdgcn_sched_barrier(0);
-        sk_block<F, TA, TU, NW, GM, MERGE, PIN>(
+        sk_block<F, TA, TU, NW, GM, MERGE, PIN, XP == 3 && F::OWN>(
             slab, wb, [&](int t) { return xl + (xb * XR + 32 * t + lr) * SK_XLD; },
             [&](int t) { return sl + (xb * XR + 32 * t + lr) * 16; }, lr, h, acc, cb, cq);
 #pragma unroll

@@ -129,8 +129,8 @@ int arfq_weight_info(const arfq_weight *w, int *qtype, int64_t *n_rows, int64_t 
  *   - m = 1: f32 x times the exact weights in f32 (Q4_K, Q5_K, IQ4_XS and Q6_K
  *     while x fits the kernels' LDS: k up to about 37K for Q4_K and 38K for the
  *     others; longer x takes the m <= 8 path below).
- *   - m <= 4: Q6_K and Q8_0 GEMVs in f32.
- *   - m <= 8 (Q4_K / Q5_K / IQ4_XS from m = 2, Q6_K / Q8_0 from m = 5): the
+ *   - m <= 4: Q6_K and Q8_0 GEMVs in f32 for small products.
+ *   - m <= 8 (Q4_K / Q5_K / IQ4_XS and larger Q6_K / Q8_0 products from m = 2): the
  *     skinny MFMA kernel with x as three f16 parts (hi + mid + lo) of x scaled
  *     per row (and per K range) by a power of two that puts the row's max |x|
  *     in [2^14, 2^15), so every x within 2^15 of that max is represented

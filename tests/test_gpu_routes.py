@@ -54,3 +54,33 @@ def test_iq4_xs_noalloc_keeps_what_fits(gpu_ctx, oracle):
     assert st == arfq.ARFQ_OK, L.arfq_last_error(gpu_ctx.handle)
     assert _rel2(y.numpy(), _want(oracle, "iq4_xs", x, raw, n)) <= 2.0 ** -11
     w.free()
+
+
+@pytest.mark.parametrize("x16", [False, True])
+@pytest.mark.parametrize("qtype,m,n,k", [
+    ("q6_k", 2, 70, 4096), ("q6_k", 4, 33, 3840), ("q6_k", 3, 40000, 256), ("q6_k", 3, 39000, 256),
+    ("q8_0", 2, 1024, 16384), ("q8_0", 2, 1023, 16384), ("q8_0", 4, 7501, 1024), ("q8_0", 4, 7200, 1024),
+    ("q8_0", 3, 4099, 4160)])
+def test_small_m_q6_k_q8_0(gpu_ctx, oracle, qtype, m, n, k, x16):
+    # both sides of the line between the f32 GEMVs and the skinny kernel (and k that only
+    # the GEMV takes): exact products everywhere, f32 sums of at most 64 block sums of 8
+    # sub-blocks, a random walk of 2^-24 steps below 2^-20.  ARFQ_OPT_GEMV_X16 has 16-bit
+    # kernels for Q6_K at m = 2 only; the rest stays exact.  Its x is off by at most half a
+    # step of 2^(e - 15), 2^e below twice the 32-element block's max, which is at most ~4
+    # times its rms: 2^-16 * 8 / sqrt(3) of x, below 2^-13.
+    _say("case: small m", qtype, m, n, k, x16)
+    raw, x = synth.weight(qtype, n, k, seed=m + n), synth.activations(m, k, seed=m + k)
+    if qtype == "q6_k":  # scales over all of i8
+        rng = np.random.default_rng(n)
+        raw.reshape(-1, 210)[:, 192:208] = rng.integers(0, 256, size=(raw.size // 210, 16), dtype=np.uint8)
+    w = gpu_ctx.upload(QType[qtype.upper()], raw, n, k)
+    y = gpu_ctx.empty((m, n), np.float32)
+    gpu_ctx.set_options(arfq.OPT_GEMV_X16 if x16 else 0)
+    try:
+        gpu_ctx.matmul(w, gpu_ctx.to_device(x), m, y)
+        got = y.numpy()
+    finally:
+        gpu_ctx.set_options(0)
+    sixteen = x16 and qtype == "q6_k" and m == 2
+    assert _rel2(got, _want(oracle, qtype, x, raw, n)) <= (2.0 ** -13 if sixteen else 2.0 ** -20)
+    w.free()
