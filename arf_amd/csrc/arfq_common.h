@@ -15,8 +15,9 @@
 //                           ggml stores element 32j+i in byte 32*(j/2)+i, low
 //                           nibble for even j, high for odd j.
 //   Q8_0  qs [nblk] 32 B  = the 32 i8 codes;   d[nblk] f16
-//   Q6_K  qb [nblk] 192 B = 4 chunks of 48 B; chunk c (n2 = c/2, l0 = 16*(c%2)):
-//                           ql[64n2+l0 .. +16] | ql[64n2+32+l0 .. +16] | qh[32n2+l0 .. +16]
+//   Q6_K  qb [nblk] 192 B = 4 chunks c (n2 = c/2, l0 = 16*(c%2)) of 48 B: ql_a, ql_b and
+//                           qh = ql[64n2+l0 .. +16], ql[64n2+32+l0 .. +16],
+//                           qh[32n2+l0 .. +16], at q6k_off(c), + Q6K_QB and + Q6K_QH
 //         sc [nblk] 16 B  = the 16 i8 sub-block scales;  d[nblk] f16
 #pragma once
 #include <hip/hip_runtime.h>
@@ -29,6 +30,9 @@ namespace arfq {
 
 constexpr int QK_K = 256;
 constexpr int WAVE = 64;
+// byte offset of a Q6_K block's chunk c (its ql_a bytes), and from there of its ql_b and qh
+__host__ __device__ constexpr int q6k_off(int c) { return 48 * c; }
+constexpr int Q6K_QB = 16, Q6K_QH = 32;
 
 // f16 bits -> f32.  v_cvt_f32_f16 is exact for every f16 value, subnormals
 // included (f16 denormals are not flushed in the default gfx950 FP mode); the
@@ -131,7 +135,7 @@ __device__ __forceinline__ float q6k_weight(float d, int sc, int q) {
 }
 
 // Extract the 6-bit code q_{t+1} (t = quadrant 0..3) of element i (0..15) of a
-// Q6_K 48-byte chunk, given the chunk as 12 dwords w[0..11]:
+// Q6_K chunk, given its ql_a, ql_b and qh bytes as 12 dwords w[0..11]:
 //   t=0: ql_a low nibble | qh bits 0-1;  t=1: ql_b low | qh bits 2-3;
 //   t=2: ql_a high       | qh bits 4-5;  t=3: ql_b high | qh bits 6-7.
 // (crates/arf-core/src/model/gguf.rs:2110-2117)

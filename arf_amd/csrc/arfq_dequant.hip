@@ -54,11 +54,11 @@ __global__ void repack_q6k(const uint8_t *__restrict__ raw, uint8_t *__restrict_
     uint8_t *dst = qb + b * 192;
     for (int c = 0; c < 4; c++) {
         const int n2 = c >> 1, l0 = 16 * (c & 1);
-        uint8_t *o = dst + 48 * c;
+        uint8_t *o = dst + q6k_off(c);
         for (int i = 0; i < 16; i++) {
             o[i] = ql[64 * n2 + l0 + i];
-            o[16 + i] = ql[64 * n2 + 32 + l0 + i];
-            o[32 + i] = qh[32 * n2 + l0 + i];
+            o[Q6K_QB + i] = ql[64 * n2 + 32 + l0 + i];
+            o[Q6K_QH + i] = qh[32 * n2 + l0 + i];
         }
     }
     int amax = 0;
@@ -154,7 +154,7 @@ __global__ void dequant_q80(const int8_t *__restrict__ qs, const uint16_t *__res
     for (int i = 0; i < 32; i++) out[b * 32 + i] = q80_weight(dv, qs[b * 32 + i]);
 }
 
-// One thread per (block, 48-byte chunk c): 64 outputs.
+// One thread per (block, chunk c): 64 outputs.
 __global__ void dequant_q6k(const uint32_t *__restrict__ qb, const int8_t *__restrict__ sc,
                             const uint16_t *__restrict__ d, float *__restrict__ out,
                             int64_t nblk) {
@@ -163,7 +163,7 @@ __global__ void dequant_q6k(const uint32_t *__restrict__ qb, const int8_t *__res
     const int64_t b = t >> 2;
     const int c = (int)(t & 3);
     uint32_t w[12];
-    for (int i = 0; i < 12; i++) w[i] = qb[b * 48 + c * 12 + i];
+    for (int i = 0; i < 12; i++) w[i] = qb[b * 48 + (i >> 2) * (Q6K_QB / 4) + q6k_off(c) / 4 + (i & 3)];
     const float dv = h2f(d[b]);
     const int n2 = c >> 1, isub = c & 1;
     float *o = out + b * 256 + 128 * n2 + 16 * isub;

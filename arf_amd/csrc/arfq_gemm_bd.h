@@ -476,10 +476,10 @@ struct BdQ6KT {
         __amdgpu_buffer_rsrc_t q, s, d;
         uint32_t qv[2], sv[2], dv[2];
         __device__ Code code(int g, int st) const {
-            const int so = (st >> 2) * 192 + 48 * (st & 3);
+            const int so = (st >> 2) * 192 + q6k_off(st & 3);
             return {__builtin_amdgcn_raw_buffer_load_b64(q, qv[g], so, 0),
-                    __builtin_amdgcn_raw_buffer_load_b64(q, qv[g] + 16, so, 0),
-                    __builtin_amdgcn_raw_buffer_load_b64(q, qv[g] + 32, so, 0)};
+                    __builtin_amdgcn_raw_buffer_load_b64(q, qv[g] + Q6K_QB, so, 0),
+                    __builtin_amdgcn_raw_buffer_load_b64(q, qv[g] + Q6K_QH, so, 0)};
         }
         __device__ Head head(int g, int blk) const {
             return {__builtin_amdgcn_raw_buffer_load_b128(s, sv[g], blk * 16, 0),

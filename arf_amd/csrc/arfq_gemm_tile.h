@@ -12,7 +12,7 @@
 //     the 16-byte LDS reads of the MFMA operands are conflict-free).
 // The next step's global loads are issued before the current step's MFMAs.
 // A step's 64 slots are one natural unit of the format (two Q4_K sub-blocks,
-// one 48-byte Q6_K chunk, two Q8_0 blocks); the x tile is gathered with the
+// one Q6_K chunk, two Q8_0 blocks); the x tile is gathered with the
 // same slot -> k permutation, so the dot product is unchanged.
 //
 // Exact weights (Q4_K, Q6_K).  The LDS tile does not hold the weights but the
@@ -166,7 +166,7 @@ struct FmtQ4K {
     }
 };
 
-// Q6_K: step st = 48-byte chunk c = st % 4 of block st / 4 (n2 = c/2,
+// Q6_K: step st = chunk c = st % 4 of block st / 4 (n2 = c/2,
 // isub = c%2); slot 16t + i is element 128*n2 + 16*isub + 32t + i (quadrant t,
 // position i).  Half ws holds positions 8ws..8ws+7 of all four quadrants.
 struct FmtQ6K {
@@ -192,11 +192,11 @@ struct FmtQ6K {
     __device__ Raw load(int64_t row, int st, int ws, int) const {
         const int64_t blk = row * nblk + (st >> 2);
         const int c = st & 3;
-        const uint2 *ch = qb8 + blk * 24 + c * 6;  // ql_a[16] | ql_b[16] | qh[16]
+        const uint2 *ch = qb8 + blk * 24 + q6k_off(c) / 8;
         Raw r;
         r.qa = ldv(ch + ws);
-        r.qb = ldv(ch + 2 + ws);
-        r.qh = ldv(ch + 4 + ws);
+        r.qb = ldv(ch + Q6K_QB / 8 + ws);
+        r.qh = ldv(ch + Q6K_QH / 8 + ws);
         r.sc = ldv(sc8 + blk * 2 + (c >> 1));  // scales 8*n2 .. 8*n2+7
         r.d = dd[blk];
         return r;

@@ -10,7 +10,8 @@
 //     codes); m = 2..4 and ARFQ_OPT_GEMV_X16: gemv_dot<Fmt> (x in 16-bit fixed
 //     point, integer dots); the same step walk; gemv_q6k is the fallback for
 //     shapes neither takes.
-//   * Q8_0: gemv_q80w, one wave per two rows, f32.
+//   * Q8_0: gemv_dot_f32 at m = 1 for large products, gemv_q80w (one wave per two
+//     rows, f32) for the rest.  m = 1 kernels take an f32 or f16 x.
 //   Large Q6_K and Q8_0 products at m = 2..4 go to the skinny MFMA kernel.
 // Reference behaviour: matmul_vec_q4ks_msl.metal:46-165 (simdgroup strides
 // sub-blocks, s*sum(q*x) + lo*sum(x) per sub-block, simd_sum), and the oracle
@@ -42,6 +43,16 @@ __device__ __forceinline__ void load16(const float *p, float *v) {
         v[4 * i + 1] = t.y;
         v[4 * i + 2] = t.z;
         v[4 * i + 3] = t.w;
+    }
+}
+
+__device__ __forceinline__ void load16(const _Float16 *p, float *v) {
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const f16x8 t = reinterpret_cast<const f16x8 *>(p)[i];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[8 * i + j] = (float)t[j];
     }
 }
 
@@ -158,6 +169,19 @@ struct XsF32 {
     const float *x;
     __device__ XqRound load(int items, int base) const { return xq_load(x, items, base); }
 };
+__device__ __forceinline__ XqRound xq_load(const _Float16 *__restrict__ x, int items, int base) {
+    const int it = min(base + (int)threadIdx.x, items - 1);
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+    const f16x8 h = reinterpret_cast<const f16x8 *>(x)[it];
+    XqRound r;
+    r.v0 = make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
+    r.v1 = make_float4((float)h[4], (float)h[5], (float)h[6], (float)h[7]);
+    return r;
+}
+struct XsF16 {
+    const _Float16 *x;
+    __device__ XqRound load(int items, int base) const { return xq_load(x, items, base); }
+};
 struct XsRowF32 {
     const float *x;
     int64_t stride;
@@ -170,15 +194,7 @@ struct XsRowF16 {
     int64_t stride;
     int div;
     __device__ void pair(int p) { x += (int64_t)(p / div) * stride; }
-    __device__ XqRound load(int items, int base) const {
-        const int it = min(base + (int)threadIdx.x, items - 1);
-        typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-        const f16x8 h = reinterpret_cast<const f16x8 *>(x)[it];
-        XqRound r;
-        r.v0 = make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
-        r.v1 = make_float4((float)h[4], (float)h[5], (float)h[6], (float)h[7]);
-        return r;
-    }
+    __device__ XqRound load(int items, int base) const { return xq_load(x, items, base); }
 };
 template <int ACT>
 struct XsGlu {
@@ -800,11 +816,11 @@ __device__ __forceinline__ void gemv_q4k_f32_body(
     }
 }
 
-template <int XR>
+template <int XR, class XSRC>
 __global__ __launch_bounds__(Q4K_F32_THREADS) void gemv_q4k_f32(
     const uint8_t *__restrict__ hdr, uint32_t hdr_bytes, const uint8_t *__restrict__ qs,
-    uint32_t qs_bytes, const float *__restrict__ x, float *__restrict__ y, int n, int nblk) {
-    gemv_q4k_f32_body<XR, Q4K_GEMV_PF, Q4K_F32_THREADS, XsF32, (XR > 1)>(hdr, hdr_bytes, qs, qs_bytes, XsF32{x}, y, n,
+    uint32_t qs_bytes, XSRC xsrc, float *__restrict__ y, int n, int nblk) {
+    gemv_q4k_f32_body<XR, Q4K_GEMV_PF, Q4K_F32_THREADS, XSRC, (XR > 1)>(hdr, hdr_bytes, qs, qs_bytes, xsrc, y, n,
                                                         nblk);
 }
 
@@ -883,7 +899,7 @@ __global__ __launch_bounds__(Q4K_GEMV_THREADS) void gemv_q4k_pairs_dual(
 // Work split as gemv_q4k: two 512-thread workgroups per CU, steps = (row,
 // column of 4 blocks) claimed in chunks of 2 rows of one column.  Lane l of a
 // 16-lane group serves block 4*column + l/4 and its 64 codes c = l%4 (four
-// 16-code quadrants); for Q6_K that is its 48-byte chunk c, one scale dword (c)
+// 16-code quadrants); for Q6_K that is its chunk c (48 bytes), one scale dword (c)
 // whose neighbours come from its quad by DPP, and the block's d.
 constexpr int Q6K_GEMV_THREADS = 512;
 constexpr int Q6K_GEMV_GROUPS = Q6K_GEMV_THREADS / 16;
@@ -943,15 +959,23 @@ __device__ __forceinline__ int q6k_subdot(const uint32_t *cw, const u32x4 lo, co
 
 // Formats of the byte-code dot GEMV.  Lane c (0..3) of a block's quad holds
 // 64 codes as four 16-code quadrants t; quadrant t's x elements start at
-// xbase(b, c) + XSTEP * t.  codes() builds the quadrant's code bytes, scales()
+// xbase(b, c) + xoff(t).  codes() builds the quadrant's code bytes, scales()
 // the per-quadrant factors, term() the quadrant's contribution from
 // sdot = sum(q * X) (X: x in 16-bit fixed point, scale xsc) and xsum = sum(x).
 //
-// Q6_K: lane c = 48-byte chunk c of the repacked block (ql_a | ql_b | qh, see
-// repack_q6k); q = ql nibble | qh bits << 4 (0..63); weight (d * sc) * (q - 32).
+// Q6_K: lane c = chunk c of the repacked block (16 bytes each of ql_a, ql_b and qh,
+// see q6k_off); q = ql nibble | qh bits << 4 (0..63); weight (d * sc) * (q - 32).
+// A load takes part of each 64-byte sector, so the loads are cached: non-temporal,
+// the sectors were fetched again for each of the three (5120 -> 151936 142.6 -> 105.7
+// us, 17408 -> 5120 20.4 -> 16.7).  Each sector read whole by one load (the block as
+// three planes) without the cache: 114 and 17.7 us.
 struct DotQ6K {
     const uint8_t *qb, *scb, *db;
-    uint32_t qb_bytes, sc_bytes, d_bytes;
+    uint32_t qb_bytes, sc_bytes, d_bytes;  // of one expert
+    __device__ DotQ6K expert(int e) const {
+        return {qb + (int64_t)e * qb_bytes, scb + (int64_t)e * sc_bytes, db + (int64_t)e * d_bytes, qb_bytes,
+                sc_bytes, d_bytes};
+    }
     struct Res {
         __amdgpu_buffer_rsrc_t q, s, d;
     };
@@ -959,17 +983,19 @@ struct DotQ6K {
         u32x4 q0, q1, q2;
         uint32_t sw, dw;
     };
-    static constexpr int XSTEP = 32, PF = Q6K_GEMV_PF;
+    static constexpr bool COLUMN = false;
+    static constexpr int PF = Q6K_GEMV_PF;
+    __device__ static int xoff(int t) { return 32 * t; }
     __device__ Res res() const {
         return {__builtin_amdgcn_make_buffer_rsrc((void *)qb, (short)0, (int)qb_bytes, 0x00020000),
                 __builtin_amdgcn_make_buffer_rsrc((void *)scb, (short)0, (int)sc_bytes, 0x00020000),
                 __builtin_amdgcn_make_buffer_rsrc((void *)db, (short)0, (int)d_bytes, 0x00020000)};
     }
     __device__ static void load(const Res &r, Lane &l, uint32_t blk, bool live, int c) {
-        const uint32_t oq = live ? blk * 192u + (uint32_t)c * 48u : Q4K_OOB;
-        l.q0 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq, 0, 2);
-        l.q1 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 16u, 0, 2);
-        l.q2 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 32u, 0, 2);
+        const uint32_t oq = live ? blk * 192u + (uint32_t)q6k_off(c) : Q4K_OOB;
+        l.q0 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq, 0, 0);
+        l.q1 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + (uint32_t)Q6K_QB, 0, 0);
+        l.q2 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + (uint32_t)Q6K_QH, 0, 0);
         l.sw = __builtin_amdgcn_raw_buffer_load_b32(r.s, live ? blk * 16u + (uint32_t)c * 4u : Q4K_OOB, 0, 0);
         l.dw = __builtin_amdgcn_raw_buffer_load_b16(r.d, live ? blk * 2u : Q4K_OOB, 0, 0);
     }
@@ -1011,6 +1037,7 @@ struct DotQ6K {
     // term; its xsum arrives as XSUM_MUL * sum(x), scaled where x is read from LDS
     static constexpr uint32_t FXOR = 0u;
     static constexpr float XSUM_MUL = -32.f;
+    static constexpr bool SIGNED = false;
     __device__ static float fterm(float A, float B, float xsc, float dot, float xsum) {
         (void)B;
         return A * __builtin_fmaf(xsc, dot, xsum);
@@ -1018,16 +1045,22 @@ struct DotQ6K {
 };
 
 // Q5_K: streams hdr (d, dmin, the 12 scale bytes: 16 B per block) and q
-// (ggml's qh[32] then qs[128]: 160 B).  Lane c takes sub-blocks 2c (low
-// nibbles of qs[32c + l]) and 2c + 1 (high nibbles), the 5th bits in qh[l] bits
-// 2c and 2c + 1; quadrant t = sub-block 2c + t / 2, elements 16 (t % 2) ..+15.
-// Each lane loads its own 32 qs bytes, a quarter of qh (bytes 8c..8c+7) and
-// header dword c; expand() gathers the whole qh and header of the block from
-// the quad by DPP, so no byte is loaded twice.  q = nibble | bit << 4 (0..31);
-// weight (d * sc) * q - dmin * m (crates/arf-core/src/model/gguf.rs:2053-2090).
+// (ggml's qh[32] then qs[128]: 160 B).  Load i (0, 1) of lane c takes qs bytes
+// 64 i + 16 c .. + 15, so a quad reads 64 contiguous bytes: with p = 2 i + c / 2
+// and l0 = 16 (c % 2), elements l0 .. + 15 of sub-blocks 2 p (low nibbles) and
+// 2 p + 1 (high), the fifth bits in bits 2 p and 2 p + 1 of qh[l0 ..].  Quadrant
+// t = sub-block 2 p + t % 2 of load t / 2.  (As 32 contiguous bytes per lane, a load
+// took 16 of every 32 bytes: 5120 -> 17408 19.0 -> 18.2 us; cached, as Q6_K's, since a
+// block's 160 bytes share 64-byte sectors with its neighbours': 16.3.)  Each lane loads a
+// quarter of qh (bytes 8c .. 8c + 7) and header dword c; expand() shares them over
+// the quad by DPP.  q = nibble | bit << 4 (0..31); weight (d * sc) * q - dmin * m
+// (crates/arf-core/src/model/gguf.rs:2053-2090).
 struct DotQ5K {
     const uint8_t *hdr, *q;
     uint32_t hdr_bytes, q_bytes;
+    __device__ DotQ5K expert(int e) const {
+        return {hdr + (int64_t)e * hdr_bytes, q + (int64_t)e * q_bytes, hdr_bytes, q_bytes};
+    }
     struct Res {
         __amdgpu_buffer_rsrc_t h, q;
     };
@@ -1035,51 +1068,55 @@ struct DotQ5K {
         u32x4 qs0, qs1;
         u32x2 qh;
         uint32_t hw;
-        uint32_t qhd[8], hd[4];  // filled by expand()
+        uint32_t qhd[4], hd[4];  // filled by expand()
     };
-    static constexpr int XSTEP = 16, PF = Q6K_GEMV_PF;
+    static constexpr int XNIB = 32;
+    static constexpr bool COLUMN = false;
+    static constexpr int PF = Q6K_GEMV_PF;
+    __device__ static int xoff(int t) { return 128 * (t >> 1) + XNIB * (t & 1); }
     __device__ Res res() const {
         return {__builtin_amdgcn_make_buffer_rsrc((void *)hdr, (short)0, (int)hdr_bytes, 0x00020000),
                 __builtin_amdgcn_make_buffer_rsrc((void *)q, (short)0, (int)q_bytes, 0x00020000)};
     }
     __device__ static void load(const Res &r, Lane &l, uint32_t blk, bool live, int c) {
         const uint32_t oq = live ? blk * 160u : Q4K_OOB;
-        l.qs0 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 32u + 32u * (uint32_t)c, 0, 2);
-        l.qs1 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 48u + 32u * (uint32_t)c, 0, 2);
-        l.qh = __builtin_amdgcn_raw_buffer_load_b64(r.q, oq + 8u * (uint32_t)c, 0, 2);
+        l.qs0 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 32u + 16u * (uint32_t)c, 0, 0);
+        l.qs1 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 96u + 16u * (uint32_t)c, 0, 0);
+        l.qh = __builtin_amdgcn_raw_buffer_load_b64(r.q, oq + 8u * (uint32_t)c, 0, 0);
         l.hw = __builtin_amdgcn_raw_buffer_load_b32(r.h, live ? blk * 16u + 4u * (uint32_t)c : Q4K_OOB, 0, 0);
     }
     __device__ static void expand(Lane &l) {
-        l.qhd[0] = quad_bcast<0>(l.qh.x), l.qhd[1] = quad_bcast<0>(l.qh.y);
-        l.qhd[2] = quad_bcast<1>(l.qh.x), l.qhd[3] = quad_bcast<1>(l.qh.y);
-        l.qhd[4] = quad_bcast<2>(l.qh.x), l.qhd[5] = quad_bcast<2>(l.qh.y);
-        l.qhd[6] = quad_bcast<3>(l.qh.x), l.qhd[7] = quad_bcast<3>(l.qh.y);
+        // qh dwords 4 (c % 2) .. + 3: lanes 2 (c % 2) and 2 (c % 2) + 1 of the quad
+        // hold two each (DPP quad_perm [0,2,0,2] and [1,3,1,3])
+        l.qhd[0] = (uint32_t)__builtin_amdgcn_mov_dpp((int)l.qh.x, 0x88, 0xf, 0xf, true);
+        l.qhd[1] = (uint32_t)__builtin_amdgcn_mov_dpp((int)l.qh.y, 0x88, 0xf, 0xf, true);
+        l.qhd[2] = (uint32_t)__builtin_amdgcn_mov_dpp((int)l.qh.x, 0xDD, 0xf, 0xf, true);
+        l.qhd[3] = (uint32_t)__builtin_amdgcn_mov_dpp((int)l.qh.y, 0xDD, 0xf, 0xf, true);
         l.hd[0] = quad_bcast<0>(l.hw), l.hd[1] = quad_bcast<1>(l.hw);
         l.hd[2] = quad_bcast<2>(l.hw), l.hd[3] = quad_bcast<3>(l.hw);
     }
-    __device__ static int xbase(int b, int c) { return 256 * b + 64 * c; }
-    // the 6-bit (sc, m) of sub-blocks 2c and 2c + 1 (q4k_scale_min without a
-    // per-lane branch)
+    __device__ static int xbase(int b, int c) { return 256 * b + 64 * (c >> 1) + 16 * (c & 1); }
+    // the 6-bit (sc, m) of sub-blocks 2 (c / 2) + {0, 1} (load 0: below 4) and those
+    // + 4 (load 1), as q4k_scale_min; byte i of the three scale dwords serves both
     __device__ static void scales(const Lane &l, int c, float A[4], float B[4]) {
         const float d = h2f(l.hd[0]), dmin = h2f(l.hd[0] >> 16);
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            const int j = 2 * c + u, i = j & 3;
+            const int i = 2 * (c >> 1) + u;
             const uint32_t a = byte_of(l.hd[1], i), bb = byte_of(l.hd[2], i), cc = byte_of(l.hd[3], i);
-            const uint32_t sc = j < 4 ? (a & 63u) : ((cc & 0xFu) | ((a >> 6) << 4));
-            const uint32_t m = j < 4 ? (bb & 63u) : ((cc >> 4) | ((bb >> 6) << 4));
-            A[2 * u] = A[2 * u + 1] = d * (float)sc;
-            B[2 * u] = B[2 * u + 1] = dmin * (float)m;
+            A[u] = d * (float)(a & 63u);
+            B[u] = dmin * (float)(bb & 63u);
+            A[2 + u] = d * (float)((cc & 0xFu) | ((a >> 6) << 4));
+            B[2 + u] = dmin * (float)((cc >> 4) | ((bb >> 6) << 4));
         }
     }
-    // quadrant t: qs bytes 16 (t % 2) + 4j ..+3 and qh dword 4 (t % 2) + j
     template <uint32_t X = 0u>
     __device__ static void codes(const Lane &l, int c, int t, uint32_t cw[4]) {
-        const int nib = t >> 1;
-        const u32x4 qs = (t & 1) ? l.qs1 : l.qs0;
+        const u32x4 qs = (t >> 1) ? l.qs1 : l.qs0;
+        const int bit = 4 * (t >> 1) + 2 * (c >> 1) + (t & 1);
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            cw[j] = (((qs[j] >> (4 * nib)) & 0x0F0F0F0Fu) | bit_to4(l.qhd[4 * (t & 1) + j], 2 * c + nib)) ^ X;
+            cw[j] = (((qs[j] >> (4 * (t & 1))) & 0x0F0F0F0Fu) | bit_to4(l.qhd[j], bit)) ^ X;
     }
     __device__ static int subdot(const uint32_t cw[4], const u32x4 lo, const u32x4 hi) {
         return q6k_subdot(cw, lo, hi);
@@ -1089,21 +1126,25 @@ struct DotQ5K {
     }
     static constexpr uint32_t FXOR = 0u;
     static constexpr float XSUM_MUL = 1.f;
+    static constexpr bool SIGNED = false;
     __device__ static float fterm(float A, float B, float xsc, float dot, float xsum) {
         return A * (xsc * dot) - B * xsum;
     }
 };
 
 // IQ4_XS: streams hdr (d, scales_h, scales_l[4]: 8 B per block) and qs (128 B).
-// Lane c takes sub-blocks 2c and 2c + 1 (qs bytes 32c .. 32c + 31); quadrant
-// t = sub-block 2c + t / 2, low (t even) or high nibbles: elements 16 t ..+15
-// of the lane's 64.  Lanes 0 and 1 load the header's two dwords and expand()
+// Load i (0, 1) of lane c takes qs bytes 64 i + 16 c .. + 15 (a quad reads 64
+// contiguous bytes; with two workgroups per CU 5120 -> 17408 17.3 -> 16.1 us), sub-block 4 i + c; quadrant t = load t / 2, low (t even) or high
+// nibbles: elements 0..15 or 16..31 of it.  Lanes 0 and 1 load the header's two dwords and expand()
 // shares them over the quad.  A code is the non-linear codebook's int8 value
 // (kvalues_iq4nl), looked up with two v_perm over the 16 entries; weight
 // (d * (ls - 32)) * kv (crates/arf-core/src/model/gguf.rs:1908-1976).
 struct DotIQ4XS {
     const uint8_t *hdr, *qs;
     uint32_t hdr_bytes, qs_bytes;
+    __device__ DotIQ4XS expert(int e) const {
+        return {hdr + (int64_t)e * hdr_bytes, qs + (int64_t)e * qs_bytes, hdr_bytes, qs_bytes};
+    }
     struct Res {
         __amdgpu_buffer_rsrc_t h, q;
     };
@@ -1112,29 +1153,31 @@ struct DotIQ4XS {
         uint32_t hw;
         uint32_t hd[2];  // filled by expand()
     };
-    static constexpr int XSTEP = 16, PF = Q6K_GEMV_PF;
+    static constexpr int XNIB = 16;
+    static constexpr bool COLUMN = false;
+    static constexpr int PF = Q6K_GEMV_PF;
+    __device__ static int xoff(int t) { return 128 * (t >> 1) + XNIB * (t & 1); }
     __device__ Res res() const {
         return {__builtin_amdgcn_make_buffer_rsrc((void *)hdr, (short)0, (int)hdr_bytes, 0x00020000),
                 __builtin_amdgcn_make_buffer_rsrc((void *)qs, (short)0, (int)qs_bytes, 0x00020000)};
     }
     __device__ static void load(const Res &r, Lane &l, uint32_t blk, bool live, int c) {
-        const uint32_t oq = live ? blk * 128u + 32u * (uint32_t)c : Q4K_OOB;
-        l.q0 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq, 0, 2);
-        l.q1 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 16u, 0, 2);
+        const uint32_t oq = live ? blk * 128u + 16u * (uint32_t)c : Q4K_OOB;
+        l.q0 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq, 0, 0);
+        l.q1 = __builtin_amdgcn_raw_buffer_load_b128(r.q, oq + 64u, 0, 0);
         l.hw = __builtin_amdgcn_raw_buffer_load_b32(r.h, live && c < 2 ? blk * 8u + 4u * (uint32_t)c : Q4K_OOB,
                                                      0, 0);
     }
     __device__ static void expand(Lane &l) {
         l.hd[0] = quad_bcast<0>(l.hw), l.hd[1] = quad_bcast<1>(l.hw);
     }
-    __device__ static int xbase(int b, int c) { return 256 * b + 64 * c; }
+    __device__ static int xbase(int b, int c) { return 256 * b + 32 * c; }
     __device__ static void scales(const Lane &l, int c, float A[4], float B[4]) {
         const float d = h2f(l.hd[0]);
-        const uint32_t sh = l.hd[0] >> 16, sl = byte_of(l.hd[1], c);
+        const uint32_t sh = l.hd[0] >> (16 + 2 * c), sl = l.hd[1] >> (4 * c);  // sub-block c; + 4: 8, 16 bits on
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            const int j = 2 * c + u;
-            const int ls = (int)(((sl >> (4 * u)) & 0xFu) | (((sh >> (2 * j)) & 3u) << 4));
+            const int ls = (int)(((sl >> (16 * u)) & 0xFu) | (((sh >> (8 * u)) & 3u) << 4));
             A[2 * u] = A[2 * u + 1] = d * (float)(ls - 32);
             B[2 * u] = B[2 * u + 1] = 0.f;
         }
@@ -1167,10 +1210,66 @@ struct DotIQ4XS {
     // f32 x: the unsigned codes kv + 128 (kv xor 0x80), less 128 * sum(x)
     static constexpr uint32_t FXOR = 0x80808080u;
     static constexpr float XSUM_MUL = -128.f;
+    static constexpr bool SIGNED = false;
     __device__ static float fterm(float A, float B, float xsc, float dot, float xsum) {
         (void)B;
         return A * __builtin_fmaf(xsc, dot, xsum);
     }
+};
+
+// Q8_0 (f32 x, k a multiple of 256: a "block" here is eight Q8_0 blocks): streams
+// qs (32 i8 codes per Q8_0 block) and d (f16).  COLUMN: a lane's quadrant t is
+// bytes 16 l .. 16 l + 15 (l = lane % 16) of block 4 column + t, so the 16 lanes
+// of a group read 256 contiguous bytes with each load.
+// The signed codes are converted as they are (SIGNED): as unsigned bytes less
+// 128 * sum(x), the error against 64 bits would grow (weight d * q,
+// matmul_nt_q8_0, crates/arf-ml/src/matmul.rs:174-204).
+struct DotQ80 {
+    const uint8_t *qs, *db;
+    uint32_t qs_bytes, d_bytes;
+    __device__ DotQ80 expert(int e) const {
+        return {qs + (int64_t)e * qs_bytes, db + (int64_t)e * d_bytes, qs_bytes, d_bytes};
+    }
+    struct Res {
+        __amdgpu_buffer_rsrc_t q, d;
+    };
+    struct Lane {
+        u32x4 q[4];
+        uint16_t d[4];
+    };
+    static constexpr bool COLUMN = true;
+    static constexpr int PF = Q6K_GEMV_PF;
+    __device__ static int xoff(int t) { return 256 * t; }
+    __device__ Res res() const {
+        return {__builtin_amdgcn_make_buffer_rsrc((void *)qs, (short)0, (int)qs_bytes, 0x00020000),
+                __builtin_amdgcn_make_buffer_rsrc((void *)db, (short)0, (int)d_bytes, 0x00020000)};
+    }
+    // blk: the column's first block, of which `live` (0..4) are within the row
+    __device__ static void load_column(const Res &r, Lane &l, uint32_t blk, int live, int l16) {
+        const uint32_t oq = blk * 256u + (uint32_t)l16 * 16u, od = blk * 16u + (uint32_t)(l16 >> 1) * 2u;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            l.q[i] = __builtin_amdgcn_raw_buffer_load_b128(r.q, i < live ? oq + 256u * i : Q4K_OOB, 0, 2);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            l.d[i] = __builtin_amdgcn_raw_buffer_load_b16(r.d, i < live ? od + 16u * i : Q4K_OOB, 0, 0);
+    }
+    __device__ static void expand(Lane &) {}
+    __device__ static int xbase(int col, int l16) { return 1024 * col + 16 * l16; }
+    // the x factor 2^(24 - s) allows for codes held as q * 2^-24; these are whole
+    __device__ static void scales(const Lane &l, int, float A[4], float *) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) A[t] = h2f(l.d[t]) * 0x1p-24f;
+    }
+    template <uint32_t X = 0u>
+    __device__ static void codes(const Lane &l, int, int t, uint32_t cw[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) cw[j] = l.q[t][j];
+    }
+    static constexpr uint32_t FXOR = 0u;
+    static constexpr float XSUM_MUL = 0.f;
+    static constexpr bool SIGNED = true;
+    __device__ static float fterm(float A, float, float xsc, float dot, float) { return A * (xsc * dot); }
 };
 
 template <class F, int MX, int XR>
@@ -1250,7 +1349,7 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot(F fmt, const float 
     }
 
     // x of the column being consumed: the lane's 4 quadrants (elements
-    // xbase + XSTEP t .. + 15)
+    // xbase + xoff(t) .. + 15)
     int xcol = -1, xbase = 0;
     u32x4 XL[4], XH[4];
     float XS[4], XE[4];
@@ -1260,7 +1359,7 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot(F fmt, const float 
         if (XREG) {
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const int eo = xbase + F::XSTEP * t;
+                const int eo = xbase + F::xoff(t);
                 XL[t] = *reinterpret_cast<const u32x4 *>(xlo + eo);
                 XH[t] = *reinterpret_cast<const u32x4 *>(xhi + eo);
                 XS[t] = s16[eo >> 4];
@@ -1291,7 +1390,7 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot(F fmt, const float 
                         xsum = XS[t];
                         xsc = XE[t];
                     } else {
-                        const size_t eo = (size_t)mi * k + xbase + F::XSTEP * t;
+                        const size_t eo = (size_t)mi * k + xbase + F::xoff(t);
                         sdot = F::subdot(cw, *reinterpret_cast<const u32x4 *>(xlo + eo),
                                          *reinterpret_cast<const u32x4 *>(xhi + eo));
                         xsum = s16[eo >> 4];
@@ -1325,7 +1424,7 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot(F fmt, const float 
     }
 }
 
-// ----------------------------------------------- Q6_K / Q5_K at f32 x (m = 1) ----
+// ------------------------- Q6_K / Q5_K / IQ4_XS / Q8_0 at f32 arithmetic (m = 1) ----
 // The dot GEMV's work split and lane map with f32 arithmetic: x is kept in LDS
 // as f32, each 32 elements scaled by 2^s (s = min(24, 100 - e), |x| < 2^e, so
 // no product overflows), with the true-unit sum of every 16 elements and
@@ -1379,9 +1478,9 @@ __device__ __forceinline__ float codes16_fdot(const uint32_t cw[4], const float 
 // narrow window of the weight stream at a time), and x is scaled into LDS
 // before the first weight load is issued (every weight request in flight
 // delays the x requests); as the Q4_K f32 GEMV (gemv_q4k_f32_body).
-template <class F, int XR>
-__global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const float *__restrict__ x,
-                                                                float *__restrict__ y, int n, int nblk) {
+template <class F, int XR, class XSRC>
+__device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc, float *__restrict__ y, int n,
+                                                  int nblk) {
     constexpr int C = Q6K_GEMV_CHUNK, PF = F::PF;
     static_assert(PF % C == 0, "claims must sit at fixed slots of the unrolled loop");
     extern __shared__ uint4 smem4[];
@@ -1457,10 +1556,16 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const fl
         } else if (u > 0) {
             irow++;
         }
-        const int b = 4 * icol + bq;
-        const bool live = icol < spr && irow < R && b < nblk;
-        const uint32_t blk = (uint32_t)(r0 + irow * G) * (uint32_t)nblk + (uint32_t)b;
-        F::load(res, ld[u], blk, live, c);
+        if constexpr (F::COLUMN) {
+            const bool live = icol < spr && irow < R;
+            const uint32_t blk = (uint32_t)(r0 + irow * G) * (uint32_t)nblk + 4u * (uint32_t)icol;
+            F::load_column(res, ld[u], blk, live ? nblk - 4 * icol : 0, l16);
+        } else {
+            const int b = 4 * icol + bq;
+            const bool live = icol < spr && irow < R && b < nblk;
+            const uint32_t blk = (uint32_t)(r0 + irow * G) * (uint32_t)nblk + (uint32_t)b;
+            F::load(res, ld[u], blk, live, c);
+        }
         srow[u] = irow;
         scol[u] = icol;
     };
@@ -1473,13 +1578,13 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const fl
     const int xitems = k / 8;
     XqRound xr[XR];
 #pragma unroll
-    for (int r = 0; r < XR; r++) xr[r] = xq_load(x, xitems, r * Q6K_GEMV_THREADS);
+    for (int r = 0; r < XR; r++) xr[r] = xsrc.load(xitems, r * Q6K_GEMV_THREADS);
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int r = 0; r < XR; r++)
         xf16_process(xr[r], xitems, r * Q6K_GEMV_THREADS, reinterpret_cast<float4 *>(xfl), s16, xe);
     for (int base = XR * Q6K_GEMV_THREADS; base < xitems; base += Q6K_GEMV_THREADS)
-        xf16_process(xq_load(x, xitems, base), xitems, base, reinterpret_cast<float4 *>(xfl), s16, xe);
+        xf16_process(xsrc.load(xitems, base), xitems, base, reinterpret_cast<float4 *>(xfl), s16, xe);
     lds_barrier();
 #pragma unroll
     for (int u = 0; u < PF; u++) issue(u, u < C);
@@ -1489,10 +1594,12 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const fl
     float X[4][16], XS[4], XE[4];
     auto load_x = [&](int col) {
         xcol = col;
-        const int xb = F::xbase(min(4 * col + bq, nblk - 1), c);
+        const int xb = F::COLUMN ? F::xbase(col, l16) : F::xbase(min(4 * col + bq, nblk - 1), c);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            const int eo = xb + F::XSTEP * t;
+            // (COLUMN: a block past the row has zero codes, and takes x = 0)
+            const bool in = !F::COLUMN || 4 * col + t < nblk;
+            const int eo = in ? xb + F::xoff(t) : 0;
             const float4 *src = reinterpret_cast<const float4 *>(xfl + eo);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -1501,6 +1608,10 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const fl
                 X[t][4 * i + 1] = v.y;
                 X[t][4 * i + 2] = v.z;
                 X[t][4 * i + 3] = v.w;
+            }
+            if constexpr (F::COLUMN) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) X[t][i] = in ? X[t][i] : 0.f;
             }
             XS[t] = F::XSUM_MUL * s16[eo >> 4];
             XE[t] = xe[eo >> 5];
@@ -1519,7 +1630,8 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const fl
         for (int t = 0; t < 4; t++) {
             uint32_t cw[4];
             F::template codes<F::FXOR>(ld[u], c, t, cw);
-            v += F::fterm(A[t], B[t], XE[t], codes16_fdot(cw, X[t]), XS[t]);
+            const float dot = F::SIGNED ? dot16_i8(X[t], make_uint4(cw[0], cw[1], cw[2], cw[3])) : codes16_fdot(cw, X[t]);
+            v += F::fterm(A[t], B[t], XE[t], dot, XS[t]);
         }
         v = row16_sum(v);
         if (l16 == 0 && live) part[(size_t)row * spr + col] = v;
@@ -1542,6 +1654,27 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const fl
     }
 }
 
+template <class F, int XR, class XSRC>
+__global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, XSRC xsrc, float *__restrict__ y, int n,
+                                                                int nblk) {
+    gemv_dot_f32_body<F, XR>(fmt, xsrc, y, n, nblk);
+}
+
+// The MoE decode pairs (as gemv_q4k_pairs): blockIdx.y = pair p, its x row times
+// the weight of expert ids[p] into y row p; blockIdx.z = 1 multiplies by a second
+// weight (the up projection beside the gate) into y1.
+template <class F, int XR, class XSRC>
+__global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_pairs(F f0, F f1, XSRC xsrc, float *__restrict__ y0,
+                                                                  float *__restrict__ y1, int n, int nblk,
+                                                                  const int32_t *__restrict__ ids, int E) {
+    const int p = blockIdx.y;
+    const int e = ids[p];
+    if (e < 0 || e >= E) return;  // uniform over the workgroup
+    const bool second = blockIdx.z != 0;
+    xsrc.pair(p);
+    gemv_dot_f32_body<F, XR>((second ? f1 : f0).expert(e), xsrc, (second ? y1 : y0) + (int64_t)p * n, n, nblk);
+}
+
 // ------------------------------------------------------------------ Q8_0 ----
 // One wave per Q80_ROWS weight rows; lane l takes blocks l, l + 64, ... of
 // each: two 16-byte code loads and the block's f16 d per row, all the loads
@@ -1552,12 +1685,14 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, const fl
 // for the wave's rows.
 // Reference arithmetic: matmul_nt_q8_0 (crates/arf-ml/src/matmul.rs:174-204).
 // two waves per workgroup (twice as many workgroups as four): C1 3.91 -> 3.73 us
-// per launch; one row per wave or four rows per wave measured 4.5-4.7 us
+// per launch; one row per wave or four rows per wave measured 4.5-4.7 us.  The loads
+// are cached: a lane's two take 16 bytes each of the same 64-byte sectors
+// (non-temporal, 8192 x 1024 5.07 against 4.67 us).
 constexpr int Q80_WAVES = 2, Q80_ROWS = 2;
-template <int MX>
+template <int MX, class XT>
 __global__ __launch_bounds__(64 * Q80_WAVES) void gemv_q80w(const uint4 *__restrict__ qs,
                                                            const uint16_t *__restrict__ dd,
-                                                           const float *__restrict__ x,
+                                                           const XT *__restrict__ x,
                                                            float *__restrict__ y, int n, int nblk,
                                                            int m) {
     constexpr int R = Q80_ROWS;
@@ -1592,8 +1727,8 @@ __global__ __launch_bounds__(64 * Q80_WAVES) void gemv_q80w(const uint4 *__restr
             if (u < nu) {
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    q[u][r][0] = ld_nt(qr[r] + 2 * bc[u]);
-                    q[u][r][1] = ld_nt(qr[r] + 2 * bc[u] + 1);
+                    q[u][r][0] = qr[r][2 * bc[u]];
+                    q[u][r][1] = qr[r][2 * bc[u] + 1];
                     dv[u][r] = h2f(dr[r][bc[u]]);
                 }
             }
@@ -1629,19 +1764,19 @@ __global__ __launch_bounds__(64 * Q80_WAVES) void gemv_q80w(const uint4 *__restr
         }
 }
 
-template <int MX>
-static hipError_t launch_q80(const arfq_weight *w, int e, int m, const float *x, float *y, hipStream_t s) {
+template <int MX, class XT>
+static hipError_t launch_q80(const arfq_weight *w, int e, int m, const XT *x, float *y, hipStream_t s) {
     const int nblk = (int)(w->k / 32);
     const int64_t eb = (int64_t)e * w->n * nblk;  // first block of expert e
     const int64_t rows_per_wg = (int64_t)Q80_WAVES * Q80_ROWS;
     const unsigned grid = (unsigned)((w->n + rows_per_wg - 1) / rows_per_wg);
-    gemv_q80w<MX><<<grid, 64 * Q80_WAVES, 0, s>>>((const uint4 *)w->s0 + eb * 2, (const uint16_t *)w->s1 + eb,
+    gemv_q80w<MX, XT><<<grid, 64 * Q80_WAVES, 0, s>>>((const uint4 *)w->s0 + eb * 2, (const uint16_t *)w->s1 + eb,
                                                   x, y, (int)w->n, nblk, m);
     return hipGetLastError();
 }
 
 // ------------------------------------------------------------------ Q6_K ----
-// Lane chunk c (0..3) of a block: 48 B = ql_a[16] | ql_b[16] | qh[16]; code i of
+// Lane chunk c (0..3) of a block: ql_a[16], ql_b[16] and qh[16]; code i of
 // quadrant t is element 128*(c/2) + 16*(c%2) + 32t + i, scale sc[8*(c/2) + c%2 + 2t].
 template <int R, int MX>
 __global__ __launch_bounds__(64) void gemv_q6k(const uint4 *__restrict__ qb,
@@ -1669,10 +1804,10 @@ __global__ __launch_bounds__(64) void gemv_q6k(const uint4 *__restrict__ qb,
             int64_t row = row0 + r;
             row = row < n ? row : n - 1;
             const int64_t blk = row * nblk + b;
-            const uint4 *src = qb + blk * 12 + c * 3;
+            const uint4 *src = qb + blk * 12 + q6k_off(c) / 16;
             w0[r] = ld_nt(src);
-            w1[r] = ld_nt(src + 1);
-            w2[r] = ld_nt(src + 2);
+            w1[r] = ld_nt(src + Q6K_QB / 16);
+            w2[r] = ld_nt(src + Q6K_QH / 16);
             // scales 8*n2 + isub + 2t, t = 0..3 -> bytes of dwords 2*n2 and 2*n2+1
             const uint32_t s_lo = scw[blk * 4 + 2 * n2], s_hi = scw[blk * 4 + 2 * n2 + 1];
             const float d = h2f(dd[blk]);
@@ -1866,6 +2001,11 @@ static DotIQ4XS dot_iq4xs(const arfq_weight *w, int e) {
     return {(const uint8_t *)w->s0 + eb * 8, (const uint8_t *)w->s1 + eb * 128, (uint32_t)(nb * 8),
             (uint32_t)(nb * 128)};
 }
+static DotQ80 dot_q80(const arfq_weight *w, int e) {
+    const int64_t nb = w->n * (w->k / 32), eb = (int64_t)e * nb;
+    return {(const uint8_t *)w->s0 + eb * 32, (const uint8_t *)w->s1 + eb * 2, (uint32_t)(nb * 32),
+            (uint32_t)(nb * 2)};
+}
 template <class F, int MX, int XR>
 static hipError_t launch_dot_t(const F &fmt, const arfq_weight *w, int m, const float *x, float *y,
                                hipStream_t s) {
@@ -1877,15 +2017,26 @@ static hipError_t launch_dot_t(const F &fmt, const arfq_weight *w, int m, const 
 // f32-x dot GEMV (m = 1): one workgroup per CU (its 137 VGPRs leave room for
 // one; held to 128 for two, it spilled and ran 31.7 us instead of 23.9 at C3)
 constexpr size_t DOT_F32_LDS_MAX = 159 * 1024;
+// below this many weights gemv_q80w: 2048 x 2048 4.5 us against 5.1 (8192 x 2048: 7.8
+// against 5.9, 17408 x 5120 33.5 against 18.6, 512 -> 100000 28.6 against 16.3)
+constexpr int64_t Q80_DOT_MIN = 12 << 20;
 static size_t dot_f32_lds_rows(const arfq_weight *w, int64_t rows) {
     const int64_t nblk = w->k / 256, spr = (nblk + 3) / 4;
     return (size_t)w->k * 4 + (size_t)(w->k / 16) * 4 + (size_t)(w->k / 32) * 4 + (size_t)rows * spr * 4;
+}
+// Workgroups per CU: one, every workgroup scaling all of x; two for IQ4_XS up to
+// k = 8192, whose codebook lookups bound it by VALU (114 VGPRs leave room for four
+// waves per SIMD), while two workgroups' x and column sums fit the LDS.
+static int dot_f32_per_cu(const arfq_weight *w) {
+    if (w->qtype != ARFQ_IQ4_XS || w->k > 8192) return 1;
+    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    return dot_f32_lds_rows(w, (w->n + 2 * cus - 1) / (2 * cus)) <= DOT_F32_LDS_MAX / 2 ? 2 : 1;
 }
 static int64_t dot_f32_grid(const arfq_weight *w) {
     const int nblk = (int)(w->k / 256);
     const int64_t steps = w->n * ((nblk + 3) / 4);
     const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
-    return std::max<int64_t>(1, std::min<int64_t>({(int64_t)cus, w->n,
+    return std::max<int64_t>(1, std::min<int64_t>({(int64_t)dot_f32_per_cu(w) * cus, w->n,
                                                    (steps + 2 * Q6K_GEMV_GROUPS - 1) / (2 * Q6K_GEMV_GROUPS)}));
 }
 static size_t dot_f32_lds(const arfq_weight *w) {
@@ -1894,21 +2045,26 @@ static size_t dot_f32_lds(const arfq_weight *w) {
 }
 static bool dot_f32_ok(const arfq_weight *w) {
     const int64_t nb = w->n * (w->k / 256);
-    const int64_t bpb = w->qtype == ARFQ_Q6_K ? 192 : w->qtype == ARFQ_Q5_K ? 160 : w->qtype == ARFQ_IQ4_XS ? 128 : 0;
+    const int64_t bpb = w->qtype == ARFQ_Q6_K ? 192 : w->qtype == ARFQ_Q5_K ? 160 : w->qtype == ARFQ_IQ4_XS ? 128
+                      : w->qtype == ARFQ_Q8_0 ? 256 : 0;
     return bpb && w->k % 256 == 0 && dot_f32_lds(w) <= DOT_F32_LDS_MAX && nb * bpb < (int64_t)Q4K_OOB &&
            (w->k / 256 + 3) / 4 <= 64;  // the kernel's column counters
 }
-template <class F, int XR>
-static hipError_t launch_dot_f32_t(const F &fmt, const arfq_weight *w, const float *x, float *y, hipStream_t s) {
+// Q8_0 at m = 1: the dot kernel where it is faster than gemv_q80w
+static bool q80_dot_m1(const arfq_weight *w) {
+    return w->qtype == ARFQ_Q8_0 && dot_f32_ok(w) && w->n * w->k >= Q80_DOT_MIN;
+}
+template <class F, int XR, class XS>
+static hipError_t launch_dot_f32_t(const F &fmt, const arfq_weight *w, const XS &x, float *y, hipStream_t s) {
     static std::atomic<uint64_t> lds_set{0};  // the attribute belongs to the kernel, per device
-    if (hipError_t err = set_max_lds_once((const void *)gemv_dot_f32<F, XR>, DOT_F32_LDS_MAX, lds_set))
+    if (hipError_t err = set_max_lds_once((const void *)gemv_dot_f32<F, XR, XS>, DOT_F32_LDS_MAX, lds_set))
         return err;
-    gemv_dot_f32<F, XR><<<(unsigned)dot_f32_grid(w), Q6K_GEMV_THREADS, dot_f32_lds(w), s>>>(
+    gemv_dot_f32<F, XR, XS><<<(unsigned)dot_f32_grid(w), Q6K_GEMV_THREADS, dot_f32_lds(w), s>>>(
         fmt, x, y, (int)w->n, (int)(w->k / 256));
     return hipGetLastError();
 }
-template <class F>
-static hipError_t launch_dot_f32(const F &fmt, const arfq_weight *w, const float *x, float *y, hipStream_t s) {
+template <class F, class XS>
+static hipError_t launch_dot_f32(const F &fmt, const arfq_weight *w, const XS &x, float *y, hipStream_t s) {
     const int64_t rounds = (w->k / 8 + Q6K_GEMV_THREADS - 1) / Q6K_GEMV_THREADS;
     if (rounds <= 1) return launch_dot_f32_t<F, 1>(fmt, w, x, y, s);
     if (rounds <= 2) return launch_dot_f32_t<F, 2>(fmt, w, x, y, s);
@@ -1994,19 +2150,20 @@ static bool q4k_f32s_ok(const arfq_weight *w) {
     return w->qtype == ARFQ_Q4_K && q4k_f32s_lds(w) <= Q4K_F32_LDS_MAX &&
            w->n * (w->k / 256) * 128 < (int64_t)Q4K_OOB && (w->k / 256 + 3) / 4 <= 64;
 }
-template <int XR>
-static hipError_t launch_q4k_f32_t(const arfq_weight *w, int e, const float *x, float *y, hipStream_t s) {
+template <int XR, class XS>
+static hipError_t launch_q4k_f32_t(const arfq_weight *w, int e, const XS &x, float *y, hipStream_t s) {
     static std::atomic<uint64_t> lds_set{0};  // the attribute belongs to the kernel, per device
-    if (hipError_t err = set_max_lds_once((const void *)gemv_q4k_f32<XR>, Q4K_F32_LDS_MAX, lds_set))
+    if (hipError_t err = set_max_lds_once((const void *)gemv_q4k_f32<XR, XS>, Q4K_F32_LDS_MAX, lds_set))
         return err;
     const int nblk = (int)(w->k / 256);
     const int64_t nb = w->n * nblk, eb = (int64_t)e * nb;
-    gemv_q4k_f32<XR><<<(unsigned)q4k_f32s_grid(w), Q4K_F32_THREADS, q4k_f32s_lds(w), s>>>(
+    gemv_q4k_f32<XR, XS><<<(unsigned)q4k_f32s_grid(w), Q4K_F32_THREADS, q4k_f32s_lds(w), s>>>(
         (const uint8_t *)w->s0 + eb * 16, (uint32_t)(nb * 16), (const uint8_t *)w->s1 + eb * 128,
         (uint32_t)(nb * 128), x, y, (int)w->n, nblk);
     return hipGetLastError();
 }
-static hipError_t launch_q4k_f32(const arfq_weight *w, int e, const float *x, float *y, hipStream_t s) {
+template <class XS>
+static hipError_t launch_q4k_f32(const arfq_weight *w, int e, const XS &x, float *y, hipStream_t s) {
     switch (q4k_f32_xr(w, Q4K_F32_THREADS)) {
     case 1: return launch_q4k_f32_t<1>(w, e, x, y, s);
     case 2: return launch_q4k_f32_t<2>(w, e, x, y, s);
@@ -2204,47 +2361,67 @@ hipError_t launch_gemv_pairs(const arfq_weight *w, int64_t P, const int32_t *ids
     return launch_pairs_t(w, P, ids, XsRowF32{(const float *)x, w->k, x_div}, y, s);
 }
 
+// The f32-arithmetic GEMVs of one x row, f32 (XsF32) or f16 (XsF16).
+template <class XS>
+static hipError_t launch_m1(const arfq_weight *w, int e, const XS &x, float *y, hipStream_t s) {
+    switch (w->qtype) {
+    case ARFQ_Q4_K:
+        return launch_q4k_f32(w, e, x, y, s);
+    case ARFQ_Q5_K:
+        return launch_dot_f32(dot_q5k(w, e), w, x, y, s);
+    case ARFQ_IQ4_XS:
+        return launch_dot_f32(dot_iq4xs(w, e), w, x, y, s);
+    case ARFQ_Q6_K:
+        if (dot_f32_ok(w)) return launch_dot_f32(dot_q6k(w, e), w, x, y, s);
+        return hipErrorInvalidValue;
+    case ARFQ_Q8_0:
+        if (q80_dot_m1(w)) return launch_dot_f32(dot_q80(w, e), w, x, y, s);
+        return launch_q80<1>(w, e, 1, x.x, y, s);
+    default:
+        return hipErrorInvalidValue;
+    }
+}
+
+bool gemv_f16_supports(const arfq_weight *w, int64_t m) {
+    if (m != 1) return false;
+    switch (w->qtype) {
+    case ARFQ_Q4_K: return q4k_f32s_ok(w);
+    case ARFQ_Q8_0: return w->k % 256 == 0;
+    default: return dot_f32_ok(w);
+    }
+}
+hipError_t launch_gemv_f16(const arfq_weight *w, int e, const void *x, float *y, hipStream_t s) {
+    if (!gemv_f16_supports(w, 1)) return hipErrorInvalidValue;
+    return launch_m1(w, e, XsF16{(const _Float16 *)x}, y, s);
+}
+
 hipError_t launch_gemv(const arfq_weight *w, int e, int64_t m, const float *x, float *y,
                        hipStream_t s, bool x16) {
     if (!gemv_supports(w, m, x16)) return hipErrorInvalidValue;
-    if (w->qtype == ARFQ_Q4_K) {
-        if (x16 && q4k_x16_ok(w, m)) {
-            if (m == 1) return launch_gemv_q4k<1>(w, e, 1, x, y, s);
-            if (m == 2) return launch_gemv_q4k<2>(w, e, 2, x, y, s);
-            return launch_gemv_q4k<4>(w, e, (int)m, x, y, s);
-        }
-        return launch_q4k_f32(w, e, x, y, s);  // m == 1, q4k_f32s_ok
+    if (x16 && q4k_x16_ok(w, m)) {
+        if (m == 1) return launch_gemv_q4k<1>(w, e, 1, x, y, s);
+        if (m == 2) return launch_gemv_q4k<2>(w, e, 2, x, y, s);
+        return launch_gemv_q4k<4>(w, e, (int)m, x, y, s);
     }
-    if (w->qtype == ARFQ_Q5_K) {
-        const DotQ5K f = dot_q5k(w, e);
-        if (x16 && dot_ok(w, m)) {
+    if (x16 && dot_ok(w, m)) {
+        if (w->qtype == ARFQ_Q5_K) {
+            const DotQ5K f = dot_q5k(w, e);
             if (m == 1) return launch_dot<DotQ5K, 1>(f, w, 1, x, y, s);
             if (m == 2) return launch_dot<DotQ5K, 2>(f, w, 2, x, y, s);
             return launch_dot<DotQ5K, 4>(f, w, (int)m, x, y, s);
         }
-        return launch_dot_f32(f, w, x, y, s);  // m == 1, dot_f32_ok
-    }
-    if (w->qtype == ARFQ_IQ4_XS) {
-        const DotIQ4XS f = dot_iq4xs(w, e);
-        if (x16 && dot_ok(w, m)) {
+        if (w->qtype == ARFQ_IQ4_XS) {
+            const DotIQ4XS f = dot_iq4xs(w, e);
             if (m == 1) return launch_dot<DotIQ4XS, 1>(f, w, 1, x, y, s);
             if (m == 2) return launch_dot<DotIQ4XS, 2>(f, w, 2, x, y, s);
             return launch_dot<DotIQ4XS, 4>(f, w, (int)m, x, y, s);
         }
-        return launch_dot_f32(f, w, x, y, s);  // m == 1, dot_f32_ok
+        const DotQ6K f = dot_q6k(w, e);
+        return m == 1 ? launch_dot<DotQ6K, 1>(f, w, 1, x, y, s) : launch_dot<DotQ6K, 2>(f, w, 2, x, y, s);
     }
-    if (w->qtype == ARFQ_Q6_K) {
-        if (x16 && dot_ok(w, m)) {
-            const DotQ6K f = dot_q6k(w, e);
-            return m == 1 ? launch_dot<DotQ6K, 1>(f, w, 1, x, y, s) : launch_dot<DotQ6K, 2>(f, w, 2, x, y, s);
-        }
-        if (m == 1 && dot_f32_ok(w)) return launch_dot_f32(dot_q6k(w, e), w, x, y, s);
-    }
-    if (w->qtype == ARFQ_Q8_0) {
-        if (m == 1) return launch_q80<1>(w, e, 1, x, y, s);
-        if (m == 2) return launch_q80<2>(w, e, 2, x, y, s);
-        return launch_q80<4>(w, e, (int)m, x, y, s);
-    }
+    if (m == 1 && (w->qtype != ARFQ_Q6_K || dot_f32_ok(w))) return launch_m1(w, e, XsF32{x}, y, s);
+    if (w->qtype == ARFQ_Q8_0)
+        return m == 2 ? launch_q80<2>(w, e, 2, x, y, s) : launch_q80<4>(w, e, (int)m, x, y, s);
     // Q6_K, f32: gemv_q6k
     if (m == 1) return launch_gemv_t<4, 1>(w, e, 1, x, y, s);
     if (m == 2) return launch_gemv_t<4, 2>(w, e, 2, x, y, s);

@@ -362,6 +362,8 @@ static int matmul_enqueue(arfq_ctx *ctx, const arfq_weight *w, int expert, int64
     const bool x16 = (ctx->options & ARFQ_OPT_GEMV_X16) != 0;
     if (x_dtype == ARFQ_F32 && arfq::gemv_supports(w, m, x16)) {
         e = arfq::launch_gemv(w, expert, m, (const float *)x, y, ctx->stream, x16);
+    } else if (x_dtype == ARFQ_F16 && arfq::gemv_f16_supports(w, m)) {
+        e = arfq::launch_gemv_f16(w, expert, x, y, ctx->stream);
     } else if (arfq::gemm_supports(w, m)) {
         const arfq::GemmPlan plan = arfq::gemm_plan(w, m, x_dtype, x16);
         if (int rc = ensure_scratch(ctx, plan.scratch_bytes)) return rc;
@@ -392,6 +394,8 @@ int arfq_matmul_noalloc(arfq_ctx *ctx, const arfq_weight *w, int expert, int64_t
     if (x_dtype == ARFQ_F32 && arfq::gemv_supports(w, m, x16)) {
         // the decode GEMVs use no scratch
         e = arfq::launch_gemv(w, expert, m, (const float *)x, y, ctx->stream, x16);
+    } else if (x_dtype == ARFQ_F16 && arfq::gemv_f16_supports(w, m)) {
+        e = arfq::launch_gemv_f16(w, expert, x, y, ctx->stream);
     } else if (arfq::gemm_supports(w, m)) {
         const arfq::GemmPlan plan = arfq::gemm_plan(w, m, x_dtype, x16, ARFQ_NOALLOC_SCRATCH_BYTES);
         if (plan.scratch_bytes > ARFQ_NOALLOC_SCRATCH_BYTES)

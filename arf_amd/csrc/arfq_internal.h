@@ -96,6 +96,9 @@ hipError_t launch_dequant(const arfq_weight *w, float *out, hipStream_t s);
 hipError_t launch_gemv(const arfq_weight *w, int e, int64_t m, const float *x, float *y,
                        hipStream_t s, bool x16 = false);
 bool gemv_supports(const arfq_weight *w, int64_t m, bool x16 = false);
+// The same for one f16 x row (m = 1), f32 arithmetic.
+bool gemv_f16_supports(const arfq_weight *w, int64_t m);
+hipError_t launch_gemv_f16(const arfq_weight *w, int e, const void *x, float *y, hipStream_t s);
 // MoE decode GEMVs over P (token, expert) pairs, Q4_K: y[p] (w->n floats) = W_ids[p] .
 // x_p, where x_p is row p / x_div of x (f32 or f16, [*, w->k]) or, when g is
 // set, silu(g[p]) * u[p] (g, u: [P, w->k] f32).  Pairs with an out-of-range id

@@ -122,7 +122,7 @@ struct SkQ4K {
     }
 };
 
-// Q6_K: step p = 48-byte chunk p (n2 = p/2, isub = p%2); lane half h takes
+// Q6_K: step p = chunk p (n2 = p/2, isub = p%2); lane half h takes
 // positions 8h .. 8h + 7 of the 4 quadrants; MFMA kk = quadrant kk:
 // element 128 n2 + 16 isub + 32 kk + 8 h + i.
 struct SkQ6K {
@@ -173,10 +173,10 @@ struct SkQ6K {
     // q - 32: v_perm puts two code bytes under 0x64 (the f16 1024 + q), less
     // 1056, exact
     __device__ static void frag(const uint8_t *srow, const Blk &, int p, int h, half8 f[4]) {
-        const uint8_t *ch = srow + 48 * p;  // ql_a[16] | ql_b[16] | qh[16]
+        const uint8_t *ch = srow + q6k_off(p);
         const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch + 8 * h);
-        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + 16 + 8 * h);
-        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + 32 + 8 * h);
+        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + Q6K_QB + 8 * h);
+        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + Q6K_QH + 8 * h);
         const half2v m1056 = h2splat(-1056.f);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -209,10 +209,10 @@ struct SkQ6KI : SkQ6K {
     __host__ __device__ SkQ6KI shifted(int64_t nb) const { return {SkQ6K::shifted(nb)}; }
     __device__ static float2 scale(const Blk &k) { return make_float2(2.f * h2f(k.d), 0.f); }
     __device__ static void frag(const uint8_t *srow, const Blk &k, int p, int h, half8 f[4]) {
-        const uint8_t *ch = srow + 48 * p;
+        const uint8_t *ch = srow + q6k_off(p);
         const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch + 8 * h);
-        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + 16 + 8 * h);
-        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + 32 + 8 * h);
+        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + Q6K_QB + 8 * h);
+        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + Q6K_QH + 8 * h);
         // scale bytes as sc + 128 (unsigned)
         const uint32_t scw[4] = {k.sc.x ^ 0x80808080u, k.sc.y ^ 0x80808080u, k.sc.z ^ 0x80808080u,
                                  k.sc.w ^ 0x80808080u};
