@@ -15,9 +15,10 @@
 //                           ggml stores element 32j+i in byte 32*(j/2)+i, low
 //                           nibble for even j, high for odd j.
 //   Q8_0  qs [nblk] 32 B  = the 32 i8 codes;   d[nblk] f16
-//   Q6_K  qb [nblk] 192 B = 4 chunks c (n2 = c/2, l0 = 16*(c%2)) of 48 B: ql_a, ql_b and
-//                           qh = ql[64n2+l0 .. +16], ql[64n2+32+l0 .. +16],
-//                           qh[32n2+l0 .. +16], at q6k_off(c), + Q6K_QB and + Q6K_QH
+//   Q6_K  qb [nblk] 192 B = per half n2 32 B each of ql_a, ql_b and qh; chunk c (n2 =
+//                           c/2, l0 = 16*(c%2)) has 16 B of each, ql[64n2+l0 .. +16],
+//                           ql[64n2+32+l0 .. +16] and qh[32n2+l0 .. +16], at
+//                           q6k_off(c), + Q6K_QB and + Q6K_QH
 //         sc [nblk] 16 B  = the 16 i8 sub-block scales;  d[nblk] f16
 #pragma once
 #include <hip/hip_runtime.h>
@@ -31,8 +32,8 @@ namespace arfq {
 constexpr int QK_K = 256;
 constexpr int WAVE = 64;
 // byte offset of a Q6_K block's chunk c (its ql_a bytes), and from there of its ql_b and qh
-__host__ __device__ constexpr int q6k_off(int c) { return 48 * c; }
-constexpr int Q6K_QB = 16, Q6K_QH = 32;
+__host__ __device__ constexpr int q6k_off(int c) { return 96 * (c >> 1) + 16 * (c & 1); }
+constexpr int Q6K_QB = 32, Q6K_QH = 64;
 
 // f16 bits -> f32.  v_cvt_f32_f16 is exact for every f16 value, subnormals
 // included (f16 denormals are not flushed in the default gfx950 FP mode); the

@@ -143,6 +143,7 @@ __device__ __forceinline__ void bd_mins(const u32x4 hd, float inv_su, int h, bf1
 // Q4_K (exact): step p, lane half h = sub-block 2p + h; group kk = code dword
 // kk (elements 8kk .. 8kk + 7, sigma nibble order).  Operands sc_j * q.
 struct BdQ4K {
+    static constexpr bool PAIR = false;
     static constexpr int XPARTS = 2;
     static constexpr bool EXTRA = false;
     struct Extra {};
@@ -206,6 +207,7 @@ struct BdQ4K {
 // f16 pattern (bit 4 of 1024 + q, bit 8 of 1024 + 16 q).  Same header and
 // min term as Q4_K.  (dequant_q5_k, crates/arf-core/src/model/gguf.rs:2053-2090)
 struct BdQ5K {
+    static constexpr bool PAIR = false;
     static constexpr int XPARTS = 4;
     static constexpr bool EXTRA = true;  // the qh bytes come separately, late
     static constexpr bool XPERM = true, LATE = true;
@@ -299,6 +301,7 @@ struct BdQ5K {
 // against 64 bits 2.1e-4 -> 1.7e-4: the tile loop rounds every weight).
 // (dequant_iq4_xs, crates/arf-core/src/model/gguf.rs:1937-1976)
 struct BdIQ4XS {
+    static constexpr bool PAIR = false;
     static constexpr int XPARTS = 2;
     static constexpr bool EXTRA = false;
     struct Extra {};
@@ -374,6 +377,7 @@ struct BdIQ4XS {
 // f16 values and hi + lo = d * q, so each group runs its MFMAs twice, once per
 // part (WLO).  (dequant_q8_0, crates/arf-core/src/model/gguf.rs)
 struct BdQ80 {
+    static constexpr bool PAIR = false;
     static constexpr int XPARTS = 2;
     static constexpr bool EXTRA = false;
     struct Extra {};
@@ -442,10 +446,16 @@ struct BdQ80 {
     }
 };
 
-// Q6_K (exact): step p = 48-byte chunk p of the block (ql_a[16] | ql_b[16] |
-// qh[16]); lane half h takes bytes 8h .. 8h + 7 of each; group kk = quadrant
-// kk: elements 128 (p / 2) + 16 (p % 2) + 32 kk + 8h + 0..7, one 16-element
-// sub-block.  Operands sc * (q - 32) in units of d: an integer of magnitude at
+// Q6_K (exact): steps 2s and 2s + 1 share chunks 2s and 2s + 1 of the block, lane
+// half h taking chunk c = 2s + h: step 2s its 16 ql_a bytes (quadrants t = 0, 2),
+// step 2s + 1 its ql_b bytes (t = 1, 3), both with its 16 qh bytes, loaded once with
+// step 2s (PAIR).  Group kk = quadrant t = p % 2 + 2 (kk / 2), positions 8 r .. 8 r + 7
+// (r = kk % 2): elements 128 s + 16 h + 32 t + 8 r + 0..7, within one 16-element
+// sub-block.  (Three 16-byte loads per two steps, the two halves' side by side: a
+// chunk per step, its halves 8 bytes each of ql_a, ql_b and qh, took six 8-byte ones;
+// 2048 x 17408 -> 5120 at f16 x 684 -> 660 us, 777 x 4096 -> 4096 at f32 x 111.5 ->
+// 106.9.  With 48 bytes per chunk 333 x 11008 -> 4096 had lost 1 % by it, with the
+// halves' bytes side by side it gains 2 %.)  Operands sc * (q - 32) in units of d: an integer of magnitude at
 // most 128 * 32 = 4096, exact in f16 up to 2048 (|sc| <= 64, the synthetic
 // scales and WIDE = false); past 2048 f16 holds only even integers, so with
 // WIDE (a tensor with some |sc| > 64) hi = sc * (q - 32) rounded and lo =
@@ -459,27 +469,32 @@ struct BdQ6KT {
     static constexpr bool XPERM = false, LATE = true;
     static constexpr bool UNITS = true, MIN = false, STEP_KK = true, WLO = WIDE;
     static constexpr int VPM = 7;
+    static constexpr bool PAIR = true;
     struct Code {
-        u32x2 a, b, qh;
+        u32x4 ql, qh;
     };
     struct Head {
         u32x4 sc;
         uint32_t d;
     };
-    using Blk = u32x4;  // the 16 int8 sub-block scales
+    using Blk = u32x4;  // the 16 int8 sub-block scales, shifted so that byte 2 i is this half's
     using Step = half2v;
     const uint2 *qb8;
     const uint4 *sc16;
     const uint16_t *dd;
-    __device__ static int a_off(int p, int kk, int h) { return 128 * (p >> 1) + 16 * (p & 1) + 32 * kk + 8 * h; }
+    __device__ static int a_off(int p, int kk, int h) {
+        return 128 * (p >> 1) + 16 * h + 32 * ((p & 1) + (kk & 2)) + 8 * (kk & 1);
+    }
     struct Lanes {
         __amdgpu_buffer_rsrc_t q, s, d;
         uint32_t qv[2], sv[2], dv[2];
-        __device__ Code code(int g, int st) const {
-            const int so = (st >> 2) * 192 + q6k_off(st & 3);
-            return {__builtin_amdgcn_raw_buffer_load_b64(q, qv[g], so, 0),
-                    __builtin_amdgcn_raw_buffer_load_b64(q, qv[g] + Q6K_QB, so, 0),
-                    __builtin_amdgcn_raw_buffer_load_b64(q, qv[g] + Q6K_QH, so, 0)};
+        // chunk 2s + h of step st: its ql_a (even steps) or ql_b bytes, its qh bytes
+        __device__ u32x4 ql(int g, int st) const {
+            return __builtin_amdgcn_raw_buffer_load_b128(
+                q, qv[g], (st >> 2) * 192 + q6k_off(st & 2) + (st & 1) * Q6K_QB, 0);
+        }
+        __device__ u32x4 qh(int g, int st) const {
+            return __builtin_amdgcn_raw_buffer_load_b128(q, qv[g], (st >> 2) * 192 + q6k_off(st & 2) + Q6K_QH, 0);
         }
         __device__ Head head(int g, int blk) const {
             return {__builtin_amdgcn_raw_buffer_load_b128(s, sv[g], blk * 16, 0),
@@ -491,8 +506,8 @@ struct BdQ6KT {
         l.q = __builtin_amdgcn_make_buffer_rsrc((void *)qb8, (short)0, (int)((uint32_t)n * nblk * 192), 0x00020000);
         l.s = __builtin_amdgcn_make_buffer_rsrc((void *)sc16, (short)0, (int)((uint32_t)n * nblk * 16), 0x00020000);
         l.d = __builtin_amdgcn_make_buffer_rsrc((void *)dd, (short)0, (int)((uint32_t)n * nblk * 2), 0x00020000);
-        l.qv[0] = wr0 * nblk * 192 + 8 * h;
-        l.qv[1] = wr1 * nblk * 192 + 8 * h;
+        l.qv[0] = wr0 * nblk * 192 + q6k_off(h);
+        l.qv[1] = wr1 * nblk * 192 + q6k_off(h);
         l.sv[0] = wr0 * nblk * 16;
         l.sv[1] = wr1 * nblk * 16;
         l.dv[0] = wr0 * nblk * 2;
@@ -500,10 +515,13 @@ struct BdQ6KT {
         return l;
     }
     __device__ static float unit(const Head &hd) { return h2f(hd.d); }
-    __device__ static Blk block(const Head &hd, const Extra &, int, uint32_t *) { return hd.sc; }
+    __device__ static Blk block(const Head &hd, const Extra &, int h, uint32_t *) {
+        return {hd.sc.x >> (8 * h), hd.sc.y >> (8 * h), hd.sc.z >> (8 * h), hd.sc.w >> (8 * h)};
+    }
     __device__ static void kill(Blk &b) { b = u32x4{0u, 0u, 0u, 0u}; }
+    // scale 8 s + h + 2 t
     __device__ static Step step(const Blk &b, int p, int kk) {
-        const int si = 8 * (p >> 1) + (p & 1) + 2 * kk;
+        const int si = 8 * (p >> 1) + 2 * ((p & 1) + (kk & 2));
         const uint32_t w = (si >> 2) == 0 ? b.x : (si >> 2) == 1 ? b.y : (si >> 2) == 2 ? b.z : b.w;
         return h2splat((float)(int8_t)(w >> (8 * (si & 3))));
     }
@@ -511,19 +529,19 @@ struct BdQ6KT {
     // qh bits go to bits 4-5), minus 1056 (exact), times sc (one rounding,
     // none while |sc| <= 64); LO: the rounding error as a second operand
     template <bool LO>
-    __device__ static void deq_t(const Code &c, const Step &sc, int kk, half8 &hi, half8 &lo) {
+    __device__ static void deq_t(const Code &c, const Step &sc, int p, int kk, half8 &hi, half8 &lo) {
         const half2v m1056 = {-1056.f, -1056.f};
-        const u32x2 ql = (kk & 1) ? c.b : c.a;
+        const int t = (p & 1) + (kk & 2);
         uint32_t o[4], e[4];
 #pragma unroll
         for (int hh = 0; hh < 2; hh++) {
-            const uint32_t l = (kk & 2) ? ((hh ? ql.y : ql.x) >> 4) : (hh ? ql.y : ql.x);
-            const uint32_t qw = hh ? c.qh.y : c.qh.x;
+            const uint32_t lw = c.ql[2 * (kk & 1) + hh], l = (kk & 2) ? lw >> 4 : lw;
+            const uint32_t qw = c.qh[2 * (kk & 1) + hh];
 #pragma unroll
             for (int pr = 0; pr < 2; pr++) {
                 const uint32_t lp = __builtin_amdgcn_perm(0x64646464u, l, pr ? 0x04030402u : 0x04010400u);
                 const uint32_t hp = __builtin_amdgcn_perm(0u, qw, pr ? 0x0c030c02u : 0x0c010c00u);
-                const uint32_t top = 2 * kk <= 4 ? (hp << (4 - 2 * kk)) : (hp >> (2 * kk - 4));
+                const uint32_t top = 2 * t <= 4 ? (hp << (4 - 2 * t)) : (hp >> (2 * t - 4));
                 const uint32_t q = (lp & 0x640F640Fu) | (top & 0x00300030u);
                 const half2v qm = as_h2(q) + m1056;
                 const half2v hv = qm * sc;
@@ -534,13 +552,13 @@ struct BdQ6KT {
         hi = bd_h8(o[0], o[1], o[2], o[3]);
         if constexpr (LO) lo = bd_h8(e[0], e[1], e[2], e[3]);
     }
-    __device__ static half8 deq(const Code &c, const Step &sc, const Blk &, int, int kk) {
+    __device__ static half8 deq(const Code &c, const Step &sc, const Blk &, int p, int kk) {
         half8 hi, lo;
-        deq_t<false>(c, sc, kk, hi, lo);
+        deq_t<false>(c, sc, p, kk, hi, lo);
         return hi;
     }
-    __device__ static void deq2(const Code &c, const Step &sc, const Blk &, int, int kk, half8 &hi, half8 &lo) {
-        deq_t<true>(c, sc, kk, hi, lo);
+    __device__ static void deq2(const Code &c, const Step &sc, const Blk &, int p, int kk, half8 &hi, half8 &lo) {
+        deq_t<true>(c, sc, p, kk, hi, lo);
     }
 };
 using BdQ6K = BdQ6KT<false>;   // every |sc| <= 64: one exact operand
@@ -660,12 +678,21 @@ __global__ __launch_bounds__(BD_THREADS, 1) void gemm_bd(
     auto xstore_at = [](int i, int q) { return XP == 2 ? i == (q == 0 ? 8 : 15) : i == (q == 3 ? 15 : 4 * q + 4); };
 
     // code ring: slot s % 2 holds step s (both groups' codes); it is refilled
-    // with step s + 2 as soon as its last operand is built
-    typename F::Code cq[2][2];
+    // with step s + 2 as soon as its last operand is built (PAIR: the qh bytes
+    // come with the even step and pass to the odd one at its first operand,
+    // before the even slot is refilled)
+    typename F::Code cq[2][2] = {};
     auto cload = [&](int u, int st) {
         st = min(st, st1 - 1);  // past the end: reload the last step (unused)
-        cq[u][0] = ld.code(0, st);
-        cq[u][1] = ld.code(1, st);
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            if constexpr (F::PAIR) {
+                if (u == 0) cq[0][g].qh = ld.qh(g, st);
+                cq[u][g].ql = ld.ql(g, st);
+            } else {
+                cq[u][g] = ld.code(g, st);
+            }
+        }
     };
     // block headers of the two rows, one block ahead; a format's EXTRA block
     // data, from group 9 of the block before
@@ -758,6 +785,12 @@ __global__ __launch_bounds__(BD_THREADS, 1) void gemm_bd(
         };
         auto deq = [&](int i, int g) {
             const int p = i >> 2, kk = i & 3;
+            if constexpr (F::PAIR) {
+                if ((p & 1) && kk == 0 && g == 0) {
+                    cq[1][0].qh = cq[0][0].qh;
+                    cq[1][1].qh = cq[0][1].qh;
+                }
+            }
             if (F::STEP_KK || kk == 0) ks[g] = F::step(scd[g], p, kk);
             if constexpr (F::WLO)
                 F::deq2(cq[p & 1][g], ks[g], scd[g], p, kk, b[g], bw[g]);
