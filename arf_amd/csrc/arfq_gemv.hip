@@ -1660,7 +1660,9 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_f32(F fmt, XSRC xsr
     gemv_dot_f32_body<F, XR>(fmt, xsrc, y, n, nblk);
 }
 
-// The MoE decode pairs (as gemv_q4k_pairs): blockIdx.y = pair p, its x row times
+// The MoE decode pairs (as gemv_q4k_pairs; one top-8 token over 128 Q4_K / Q6_K experts
+// 75.8 us in the grouped kernels, whose tiles hold a row or two, 22.5 here; arfq_host.hip
+// says up to how many pairs): blockIdx.y = pair p, its x row times
 // the weight of expert ids[p] into y row p; blockIdx.z = 1 multiplies by a second
 // weight (the up projection beside the gate) into y1.
 template <class F, int XR, class XSRC>
@@ -2043,11 +2045,15 @@ static size_t dot_f32_lds(const arfq_weight *w) {
     const int64_t g = dot_f32_grid(w);
     return dot_f32_lds_rows(w, (w->n + g - 1) / g);
 }
-static bool dot_f32_ok(const arfq_weight *w) {
+// a dot format whose largest stream (of one expert) fits 31-bit buffer offsets
+static bool dot_stream_ok(const arfq_weight *w) {
     const int64_t nb = w->n * (w->k / 256);
     const int64_t bpb = w->qtype == ARFQ_Q6_K ? 192 : w->qtype == ARFQ_Q5_K ? 160 : w->qtype == ARFQ_IQ4_XS ? 128
                       : w->qtype == ARFQ_Q8_0 ? 256 : 0;
-    return bpb && w->k % 256 == 0 && dot_f32_lds(w) <= DOT_F32_LDS_MAX && nb * bpb < (int64_t)Q4K_OOB &&
+    return bpb && w->k % 256 == 0 && nb * bpb < (int64_t)Q4K_OOB;
+}
+static bool dot_f32_ok(const arfq_weight *w) {
+    return dot_stream_ok(w) && dot_f32_lds(w) <= DOT_F32_LDS_MAX &&
            (w->k / 256 + 3) / 4 <= 64;  // the kernel's column counters
 }
 // Q8_0 at m = 1: the dot kernel where it is faster than gemv_q80w
@@ -2224,23 +2230,65 @@ hipError_t launch_gemv_dual(const arfq_weight *a, const arfq_weight *b, const fl
 // LDS of gemv_q4k_pairs with g workgroups per pair.
 static size_t q4k_pairs_lds(const arfq_weight *w, int64_t g) { return q4k_f32_lds_rows(w, (w->n + g - 1) / g); }
 
-bool gemv_pairs_supports(const arfq_weight *w) {
-    return w->qtype == ARFQ_Q4_K && w->k % 256 == 0 && w->n * (w->k / 256) * 128 < (int64_t)Q4K_OOB &&
-           q4k_pairs_lds(w, 1) <= Q4K_F32_LDS_MAX && (w->k / 256 + 3) / 4 <= 64;
-}
-
 // Workgroups per CU of the decode-pair GEMVs: two, or one for up to 8 pairs (one token's
 // top-8: C5's experts at T = 1 ran 21.9 us against 23.2 with two, while at T = 4 and 16
 // one per CU was 9 % and 13 % slower).
 static int pairs_per_cu(int64_t P) { return P <= 8 ? 1 : 2; }
+// Workgroups per pair and weight, nz weights in the launch: about that many per CU over
+// all of them, >= 4 rows each.
+static int64_t pairs_grid(const arfq_weight *w, int64_t P, int nz) {
+    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    return std::max<int64_t>(1, std::min<int64_t>((pairs_per_cu(P) * (int64_t)cus + nz * P - 1) / (nz * P), w->n / 4));
+}
+static size_t dot_pairs_lds(const arfq_weight *w, int64_t g) { return dot_f32_lds_rows(w, (w->n + g - 1) / g); }
+
+bool gemv_pairs_supports(const arfq_weight *w, int64_t P, int nz) {
+    if (w->k % 256 != 0 || (w->k / 256 + 3) / 4 > 64 || P < 1 || P > 65535) return false;
+    if (w->qtype == ARFQ_Q4_K)
+        return w->n * (w->k / 256) * 128 < (int64_t)Q4K_OOB && q4k_pairs_lds(w, 1) <= Q4K_F32_LDS_MAX;
+    return dot_stream_ok(w) && dot_pairs_lds(w, pairs_grid(w, P, nz)) <= DOT_F32_LDS_MAX;
+}
+
+// The dot formats' pairs: y0 row p = W0_ids[p] . x_p and, with w1 (same qtype and
+// shape), y1 row p = W1_ids[p] . x_p in the same launch.
+template <class F, class XS>
+static hipError_t launch_dot_pairs_f(const F &f0, const F &f1, const arfq_weight *w, int nz, int64_t P,
+                                     const int32_t *ids, const XS &xs, float *y0, float *y1, hipStream_t s) {
+    const int64_t g = pairs_grid(w, P, nz);
+    const dim3 grid((unsigned)g, (unsigned)P, (unsigned)nz);
+    const size_t lds = dot_pairs_lds(w, g);
+    auto go = [&](auto kern) -> hipError_t {
+        static std::atomic<uint64_t> lds_set{0};
+        if (hipError_t err = set_max_lds_once((const void *)kern, DOT_F32_LDS_MAX, lds_set)) return err;
+        kern<<<grid, Q6K_GEMV_THREADS, lds, s>>>(f0, f1, xs, y0, y1, (int)w->n, (int)(w->k / 256), ids, w->experts);
+        return hipGetLastError();
+    };
+    return w->k <= Q6K_GEMV_THREADS * 8 ? go(gemv_dot_pairs<F, 1, XS>) : go(gemv_dot_pairs<F, 2, XS>);
+}
+template <class XS>
+static hipError_t launch_dot_pairs(const arfq_weight *w0, const arfq_weight *w1, int64_t P, const int32_t *ids,
+                                   const XS &xs, float *y0, float *y1, hipStream_t s) {
+    const int nz = w1 ? 2 : 1;
+    const arfq_weight *wb = w1 ? w1 : w0;
+    switch (w0->qtype) {
+    case ARFQ_Q5_K:
+        return launch_dot_pairs_f(dot_q5k(w0, 0), dot_q5k(wb, 0), w0, nz, P, ids, xs, y0, y1, s);
+    case ARFQ_Q6_K:
+        return launch_dot_pairs_f(dot_q6k(w0, 0), dot_q6k(wb, 0), w0, nz, P, ids, xs, y0, y1, s);
+    case ARFQ_Q8_0:
+        return launch_dot_pairs_f(dot_q80(w0, 0), dot_q80(wb, 0), w0, nz, P, ids, xs, y0, y1, s);
+    case ARFQ_IQ4_XS:
+        return launch_dot_pairs_f(dot_iq4xs(w0, 0), dot_iq4xs(wb, 0), w0, nz, P, ids, xs, y0, y1, s);
+    default:
+        return hipErrorInvalidValue;
+    }
+}
 
 template <class XS>
 static hipError_t launch_pairs_t(const arfq_weight *w, int64_t P, const int32_t *ids, const XS &xs,
                                  float *y, hipStream_t s) {
-    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
-    // about two workgroups per CU over all pairs (one at a single token's pairs), >= 4 rows
-    // per workgroup
-    const int64_t g = std::max<int64_t>(1, std::min<int64_t>((pairs_per_cu(P) * (int64_t)cus + P - 1) / P, w->n / 4));
+    if (w->qtype != ARFQ_Q4_K) return launch_dot_pairs(w, nullptr, P, ids, xs, y, y, s);
+    const int64_t g = pairs_grid(w, P, 1);
     const int64_t nb = w->n * (w->k / 256);
     const dim3 grid((unsigned)g, (unsigned)P);
     const int nsub = (int)(w->k / 32);
@@ -2315,11 +2363,8 @@ hipError_t launch_gemv_glu(const arfq_weight *w, int64_t m, const float *g, cons
 template <class XS>
 static hipError_t launch_pairs_dual_t(const arfq_weight *w0, const arfq_weight *w1, int64_t P,
                                       const int32_t *ids, const XS &xs, float *y0, float *y1, hipStream_t s) {
-    const int cus = w0->ctx->cus > 0 ? w0->ctx->cus : 256;
-    // about two workgroups per CU over both weights' pairs (one at a single token's pairs),
-    // >= 4 rows per workgroup
-    const int64_t g = std::max<int64_t>(
-        1, std::min<int64_t>((pairs_per_cu(P) * (int64_t)cus + 2 * P - 1) / (2 * P), w0->n / 4));
+    if (w0->qtype != ARFQ_Q4_K) return launch_dot_pairs(w0, w1, P, ids, xs, y0, y1, s);
+    const int64_t g = pairs_grid(w0, P, 2);
     const int64_t nb = w0->n * (w0->k / 256);
     const dim3 grid((unsigned)g, (unsigned)P, 2);
     const size_t lds = q4k_pairs_lds(w0, g);
@@ -2336,15 +2381,15 @@ static hipError_t launch_pairs_dual_t(const arfq_weight *w0, const arfq_weight *
     return go(gemv_q4k_pairs_dual<2, XS>);
 }
 
-bool gemv_pairs_dual_supports(const arfq_weight *w0, const arfq_weight *w1) {
-    return gemv_pairs_supports(w0) && gemv_pairs_supports(w1) && w1->qtype == w0->qtype &&
+bool gemv_pairs_dual_supports(const arfq_weight *w0, const arfq_weight *w1, int64_t P) {
+    return gemv_pairs_supports(w0, P, 2) && gemv_pairs_supports(w1, P, 2) && w1->qtype == w0->qtype &&
            w1->n == w0->n && w1->k == w0->k && w1->experts == w0->experts;
 }
 
 hipError_t launch_gemv_pairs_dual(const arfq_weight *w0, const arfq_weight *w1, int64_t P, const int32_t *ids,
                                   const void *x, int x_dtype, int x_div, float *y0, float *y1, hipStream_t s) {
     if (P == 0) return hipSuccess;
-    if (!gemv_pairs_dual_supports(w0, w1) || P > 65535) return hipErrorInvalidValue;
+    if (!gemv_pairs_dual_supports(w0, w1, P)) return hipErrorInvalidValue;
     if (x_dtype == ARFQ_F16)
         return launch_pairs_dual_t(w0, w1, P, ids, XsRowF16{(const _Float16 *)x, w0->k, x_div}, y0, y1, s);
     return launch_pairs_dual_t(w0, w1, P, ids, XsRowF32{(const float *)x, w0->k, x_div}, y0, y1, s);
@@ -2354,7 +2399,7 @@ hipError_t launch_gemv_pairs(const arfq_weight *w, int64_t P, const int32_t *ids
                              int x_dtype, int x_div, const float *g, const float *u, float *y,
                              hipStream_t s) {
     if (P == 0) return hipSuccess;
-    if (!gemv_pairs_supports(w) || P > 65535) return hipErrorInvalidValue;
+    if (!gemv_pairs_supports(w, P, 1)) return hipErrorInvalidValue;
     if (g) return launch_pairs_t(w, P, ids, XsSwiglu{g, u, w->k}, y, s);
     if (x_dtype == ARFQ_F16)
         return launch_pairs_t(w, P, ids, XsRowF16{(const _Float16 *)x, w->k, x_div}, y, s);

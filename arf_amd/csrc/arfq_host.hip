@@ -11,6 +11,7 @@
 #include "arfq_internal.h"
 
 #include <algorithm>
+#include <cmath>
 
 // ---- scratch of the allocation-free matmul (arfq_matmul_noalloc) ----
 // One fixed array per GPU, in the library's code object: resident from the
@@ -477,6 +478,25 @@ static int check_moe(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight *
     return ARFQ_OK;
 }
 
+// Whether P pairs run faster as GEMVs, each reading its expert's weights, than in the
+// grouped kernels, which read an expert once.  The two times in us, from MB: the GEMVs
+// 18 + 5.8 MB/us (3.3 for IQ4_XS's codebook) over every pair, the grouped kernels 55 +
+// 4.5 MB/us over the experts that some pair picks.  Measured (GEMVs / grouped): Q4_K +
+// Q6_K, 3.1 MB an expert, 128 experts, 8 / 32 / 64 / 128 pairs 22.5 / 75.8, 35.8 / 77.4,
+// 52 / 98, 86 / 108; 32 experts, 128 pairs 72 / 58; Q8_0, 6.7 MB, 64 experts, 16 / 64
+// pairs 40 / 58, 85 / 95; Q5_K + Q6_K, 22 MB, 8 experts, 10 / 32 pairs 77 / 94, 128 /
+// 96; IQ4_XS, 5.9 MB, 64 experts, 56 pairs 116 / 123; 13.6 MB, 16 experts, 96 pairs
+// 413 / 119.  Q4_K throughout always takes them: f32 arithmetic is what it has had.
+static bool moe_pairs_pay(const arfq_weight *gate, const arfq_weight *down, int64_t P) {
+    if (gate->qtype == ARFQ_Q4_K && down->qtype == ARFQ_Q4_K) return true;
+    const double E = gate->experts, w = (double)gate->n * gate->k * 1e-6;  // million weights
+    auto mb = [&](const arfq_weight *t) { return w * arfq::block_bytes_of(t->qtype) / arfq::qk_of(t->qtype); };
+    auto rate = [](const arfq_weight *t) { return t->qtype == ARFQ_IQ4_XS ? 3.3 : 5.8; };
+    const double touched = E * (1.0 - std::pow(1.0 - 1.0 / E, (double)P));
+    const double pairs = 18.0 + (double)P * (2.0 * mb(gate) / rate(gate) + mb(down) / rate(down));
+    return 1.1 * pairs < 55.0 + touched * (2.0 * mb(gate) + mb(down)) / 4.5;
+}
+
 // Route (when ids == NULL) + group + grouped GEMMs + combine, all on the stream.
 // Scratch layout: [x f16] [ids] [weights] [off] [sorted] [tiles] [ntiles] [h f16] [o f32].
 static int moe_enqueue(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight *up,
@@ -490,8 +510,8 @@ static int moe_enqueue(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight
     // gate -> up -> down with SwiGLU on its x -> combine), instead of grouping pairs
     // into expert tiles the grouped GEMMs would mostly leave empty (the reference's
     // mul_mv_id crossover, crates/arf-gpu/src/gpu/metal/island.rs:4048-4070).
-    if (P <= arfq::MOE_DECODE_PAIRS_MAX && gate->qtype == ARFQ_Q4_K && down->qtype == ARFQ_Q4_K &&
-        arfq::gemv_pairs_supports(gate) && arfq::gemv_pairs_supports(down)) {
+    if (P <= arfq::MOE_DECODE_PAIRS_MAX && arfq::gemv_pairs_supports(gate, P, 2) &&
+        arfq::gemv_pairs_supports(up, P, 2) && arfq::gemv_pairs_supports(down, P, 1) && moe_pairs_pay(gate, down, P)) {
         size_t o = 0;
         const size_t o_ids = o;  o += ids_in ? 0 : align256((size_t)P * 4);
         const size_t o_w = o;    o += ids_in ? 0 : align256((size_t)P * 4);
@@ -511,7 +531,7 @@ static int moe_enqueue(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight
             wts = (const float *)(sc + o_w);
         }
         float *g = (float *)(sc + o_g), *u = (float *)(sc + o_u), *ob = (float *)(sc + o_o);
-        if (arfq::gemv_pairs_dual_supports(gate, up)) {
+        if (arfq::gemv_pairs_dual_supports(gate, up, P)) {
             e = arfq::launch_gemv_pairs_dual(gate, up, P, ids, x, x_dtype, top_k, g, u, ctx->stream);
         } else {
             e = arfq::launch_gemv_pairs(gate, P, ids, x, x_dtype, top_k, nullptr, nullptr, g, ctx->stream);

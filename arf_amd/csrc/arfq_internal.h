@@ -99,7 +99,7 @@ bool gemv_supports(const arfq_weight *w, int64_t m, bool x16 = false);
 // The same for one f16 x row (m = 1), f32 arithmetic.
 bool gemv_f16_supports(const arfq_weight *w, int64_t m);
 hipError_t launch_gemv_f16(const arfq_weight *w, int e, const void *x, float *y, hipStream_t s);
-// MoE decode GEMVs over P (token, expert) pairs, Q4_K: y[p] (w->n floats) = W_ids[p] .
+// MoE decode GEMVs over P (token, expert) pairs: y[p] (w->n floats) = W_ids[p] .
 // x_p, where x_p is row p / x_div of x (f32 or f16, [*, w->k]) or, when g is
 // set, silu(g[p]) * u[p] (g, u: [P, w->k] f32).  Pairs with an out-of-range id
 // are skipped.
@@ -115,12 +115,13 @@ hipError_t launch_gemv_dual(const arfq_weight *a, const arfq_weight *b, const fl
                             hipStream_t s);
 // h = act(g) * u elementwise (n floats; act ARFQ_ACT_*)
 hipError_t launch_glu(const float *g, const float *u, float *h, int64_t n, int act, hipStream_t s);
-bool gemv_pairs_supports(const arfq_weight *w);
+// (nz: the weights multiplied in one launch, 1 or 2)
+bool gemv_pairs_supports(const arfq_weight *w, int64_t P, int nz);
 hipError_t launch_gemv_pairs(const arfq_weight *w, int64_t P, const int32_t *ids, const void *x,
                              int x_dtype, int x_div, const float *g, const float *u, float *y,
                              hipStream_t s);
 // MoE decode gate and up in one launch (same qtype, shape and expert count).
-bool gemv_pairs_dual_supports(const arfq_weight *w0, const arfq_weight *w1);
+bool gemv_pairs_dual_supports(const arfq_weight *w0, const arfq_weight *w1, int64_t P);
 hipError_t launch_gemv_pairs_dual(const arfq_weight *w0, const arfq_weight *w1, int64_t P, const int32_t *ids,
                                   const void *x, int x_dtype, int x_div, float *y0, float *y1, hipStream_t s);
 

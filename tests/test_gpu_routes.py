@@ -123,3 +123,39 @@ def test_m1_q8_0_infinite_x(gpu_ctx, oracle):
     fine = ~np.isnan(want)
     assert np.array_equal(y.numpy()[0][fine], want[fine])
     w.free()
+
+
+@pytest.mark.parametrize("qg,qd,tokens,top_k,hidden,inter", [
+    ("q4_k", "q6_k", 1, 2, 256, 512), ("q5_k", "q5_k", 3, 2, 768, 256), ("iq4_xs", "q6_k", 2, 3, 512, 1280),
+    ("q8_0", "q8_0", 5, 1, 1280, 512), ("q6_k", "q4_k", 4, 2, 512, 768), ("iq4_xs", "iq4_xs", 1, 4, 4352, 256),
+    ("q5_k", "q6_k", 70, 2, 512, 512), ("q8_0", "iq4_xs", 66, 2, 256, 256)])
+@pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
+def test_moe_pairs_and_grouped(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, inter, x_dtype):
+    # up to 128 pairs: the f32 GEMVs (each product's sums below 2^-20, g and u through
+    # silu(g) * u and the down sums: four such errors, 2^-18).  More pairs: the grouped
+    # kernels, x and h in f16 (2^-11 each).  One id of the given ones is out of range and
+    # adds nothing.
+    _say("case: moe", qg, qd, tokens, top_k, hidden, inter, np.dtype(x_dtype).name)
+    E = 4
+    shapes = [(qg, inter, hidden), (qg, inter, hidden), (qd, hidden, inter)]
+    raw = [synth.weight(q, n, k, seed=50 + i, experts=E) for i, (q, n, k) in enumerate(shapes)]
+    ws = [gpu_ctx.upload(QType[q.upper()], r, n, k, E) for (q, n, k), r in zip(shapes, raw)]
+    dq = [oracle.dequant(q, r, E * n * k).reshape(E, n, k).astype(np.float64) for (q, n, k), r in zip(shapes, raw)]
+    rng = np.random.default_rng(tokens)
+    x = (synth.activations(tokens, hidden, seed=7) * 0.05).astype(x_dtype)
+    ids = rng.integers(0, E, size=(tokens, top_k)).astype(np.int32)
+    wts = rng.random((tokens, top_k), dtype=np.float32)
+    ids[-1, -1] = E
+    y = gpu_ctx.empty((tokens, hidden), np.float32)
+    gpu_ctx.moe_ids(*ws, gpu_ctx.to_device(ids), gpu_ctx.to_device(wts), tokens, top_k, gpu_ctx.to_device(x), y)
+    want = np.zeros((tokens, hidden))
+    for t in range(tokens):
+        for e, wt in zip(ids[t], wts[t]):
+            if e < E:
+                g, u = dq[0][e] @ x[t].astype(np.float64), dq[1][e] @ x[t].astype(np.float64)
+                with np.errstate(over="ignore"):
+                    want[t] += wt * (dq[2][e] @ (g / (1 + np.exp(-g)) * u))
+    got = y.numpy()
+    assert _rel2(got, want) <= (2.0 ** -18 if tokens * top_k <= 128 else 2.0 ** -10)
+    for w in ws:
+        w.free()
