@@ -555,7 +555,7 @@ __global__ __launch_bounds__(DXS_THREADS, 1) void moe_down_xs_kernel(
 #pragma unroll
         for (int i = 0; i < NI; i++) {
             const int c = 64 * i + lane;
-            *reinterpret_cast<u32x4 *>(slab + (c / RL) * SL + 16 * (c % RL)) = r[i];
+            *reinterpret_cast<u32x4 *>(slab + (c / RL) * SL + 16 * slab_unit<F>(c % RL)) = r[i];
         }
     };
     auto loop = [&](auto tu) {

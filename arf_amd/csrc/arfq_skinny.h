@@ -33,6 +33,8 @@
 #pragma once
 #include "arfq_gemm_tile.h"
 
+#include <type_traits>
+
 namespace arfq {
 
 constexpr int SK_THREADS = 256;
@@ -148,6 +150,15 @@ struct SkQ6K {
     __device__ const uint8_t *raw(int64_t row, int b) const {
         return reinterpret_cast<const uint8_t *>(qb8 + (row * nblk + b) * 24);
     }
+    // The slab holds the block as chunks of 48 bytes, ql_a | ql_b | qh: 16-byte unit u
+    // of the stream (see q6k_off) goes to unit slab_unit(u).  (In the stream's own
+    // order the reads of two steps look alike to the compiler, which merges them and
+    // holds both steps' bytes: the kernel of m = 17..32 spilled and a product there took
+    // 302 us instead of 199.)
+    __device__ static int slab_unit(int u) {
+        const int n2 = u >= 6, v = u - 6 * n2;
+        return 6 * n2 + 3 * (v & 1) + (v >> 1);
+    }
     __device__ Blk load_blk(int64_t row, int b) const {
         return {ldv(sc16 + row * nblk + b), dd[row * nblk + b]};
     }
@@ -173,10 +184,10 @@ struct SkQ6K {
     // q - 32: v_perm puts two code bytes under 0x64 (the f16 1024 + q), less
     // 1056, exact
     __device__ static void frag(const uint8_t *srow, const Blk &, int p, int h, half8 f[4]) {
-        const uint8_t *ch = srow + q6k_off(p);
+        const uint8_t *ch = srow + 48 * p;
         const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch + 8 * h);
-        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + Q6K_QB + 8 * h);
-        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + Q6K_QH + 8 * h);
+        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + 16 + 8 * h);
+        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + 32 + 8 * h);
         const half2v m1056 = h2splat(-1056.f);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -209,10 +220,10 @@ struct SkQ6KI : SkQ6K {
     __host__ __device__ SkQ6KI shifted(int64_t nb) const { return {SkQ6K::shifted(nb)}; }
     __device__ static float2 scale(const Blk &k) { return make_float2(2.f * h2f(k.d), 0.f); }
     __device__ static void frag(const uint8_t *srow, const Blk &k, int p, int h, half8 f[4]) {
-        const uint8_t *ch = srow + q6k_off(p);
+        const uint8_t *ch = srow + 48 * p;
         const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch + 8 * h);
-        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + Q6K_QB + 8 * h);
-        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + Q6K_QH + 8 * h);
+        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + 16 + 8 * h);
+        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + 32 + 8 * h);
         // scale bytes as sc + 128 (unsigned)
         const uint32_t scw[4] = {k.sc.x ^ 0x80808080u, k.sc.y ^ 0x80808080u, k.sc.z ^ 0x80808080u,
                                  k.sc.w ^ 0x80808080u};
@@ -418,6 +429,16 @@ struct SkRows {
     int64_t x[XC];  // element offset (row * K) of row (tid >> 5) + (NT / 32) i
     int64_t s;      // element offset (row * K / 16) of row min(tid >> 1, XR - 1)
 };
+
+// Where 16-byte unit u of a weight row's block lies in the row's slab: as it comes, but
+// for Q6_K's chunks.
+template <class F>
+__device__ __forceinline__ int slab_unit(int u) {
+    if constexpr (std::is_base_of_v<SkQ6K, F>)
+        return F::slab_unit(u);
+    else
+        return u;
+}
 
 // LDS of the loop: XB buffers of the x block of XR rows (+ its sub-block sums)
 // and one weight slab [32][RB + 16] per wave and weight.
@@ -693,7 +714,7 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
 #pragma unroll
             for (int i = 0; i < NI; i++) {
                 const int c = 64 * i + lane;
-                *reinterpret_cast<u32x4 *>(slab + (w * 32 + c / RL) * SL + 16 * (c % RL)) = rv[w][i];
+                *reinterpret_cast<u32x4 *>(slab + (w * 32 + c / RL) * SL + 16 * slab_unit<F>(c % RL)) = rv[w][i];
             }
     };
     int64_t myrow[NW];
