@@ -347,7 +347,8 @@ static GemmPlan gemm_plan_of(const arfq_weight *w, int64_t m, int x_dtype, bool 
     const int64_t bdb = bd_stream_bytes(w->qtype);
     // (an f32 x enters it as hi + lo rows unless x16: twice the x bytes)
     const int64_t bdx = x_dtype == ARFQ_F32 && !x16 ? 2 : 1;
-    p.bd = direct && !p.skinny && m > 64 && bdb && w->k % 256 == 0 && w->n * (w->k / 256) * bdb < ((int64_t)1 << 31) && bdx * m * w->k * 2 < ((int64_t)1 << 31);  // buffer loads
+    p.bd = direct && !p.skinny && m > 64 && bdb && w->k % 256 == 0 &&
+           w->n * (w->k / 256) * bdb < ((int64_t)1 << 31) && bdx * m * w->k * 2 < ((int64_t)1 << 31);  // buffer loads
     // f32 x: scaled per row by a power of two into f16 range, then split into
     // f16 parts for the skinny kernel and the direct-operand prefill (hi + lo
     // rows: its tiles cover 64 rows at twice the MFMAs; one f16 part under x16),
@@ -450,6 +451,8 @@ static hipError_t launch_sk_t(const F &fmt, const arfq_weight *w, int64_t m, con
     if constexpr (F::KIND >= 3 && TA == 1 && GM == 0xFF) {
         // at most 8 rows (8 hi + 8 lo with two parts, + 8 mid with three): the
         // per-sub-block scaling touches only the accumulator groups that hold them
+        if constexpr (F::KIND == 4 && PARTS == 3)
+            if (m <= 4) return launch_sk_t<F, 1, 3, 0x7 | SK_OWN, XT>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
         if (m <= 8)
             return launch_sk_t<F, 1, PARTS, PARTS == 3 ? 0x7 : PARTS == 2 ? 0x5 : 0x1, XT>(fmt, w, m, x, xs, rs, rss,
                                                                                           y, part, S, s);

@@ -1134,8 +1134,9 @@ struct DotQ5K {
 
 // IQ4_XS: streams hdr (d, scales_h, scales_l[4]: 8 B per block) and qs (128 B).
 // Load i (0, 1) of lane c takes qs bytes 64 i + 16 c .. + 15 (a quad reads 64
-// contiguous bytes; with two workgroups per CU 5120 -> 17408 17.3 -> 16.1 us), sub-block 4 i + c; quadrant t = load t / 2, low (t even) or high
-// nibbles: elements 0..15 or 16..31 of it.  Lanes 0 and 1 load the header's two dwords and expand()
+// contiguous bytes; with two workgroups per CU 5120 -> 17408 17.3 -> 16.1 us),
+// sub-block 4 i + c; quadrant t = load t / 2, low (t even) or high nibbles: elements
+// 0..15 or 16..31 of it.  Lanes 0 and 1 load the header's two dwords and expand()
 // shares them over the quad.  A code is the non-linear codebook's int8 value
 // (kvalues_iq4nl), looked up with two v_perm over the 16 entries; weight
 // (d * (ls - 32)) * kv (crates/arf-core/src/model/gguf.rs:1908-1976).

@@ -132,7 +132,7 @@ struct SkQ6K {
     // 16-element sub-block, whose product is scaled by its own d * sc in f32
     // (KIND 4)
     static constexpr int KIND = 4, RB = 192;
-    static constexpr bool OWN = false;
+    static constexpr bool OWN = true;
     struct Blk {
         u32x4 sc;  // the 16 i8 scales
         uint32_t d;
@@ -430,6 +430,8 @@ struct SkRows {
     int64_t s;      // element offset (row * K / 16) of row min(tid >> 1, XR - 1)
 };
 
+constexpr int SK_OWN = 0x100;  // a bit of GM: KIND 4 sums each block apart
+
 // Where 16-byte unit u of a weight row's block lies in the row's slab: as it comes, but
 // for Q6_K's chunks.
 template <class F>
@@ -454,11 +456,12 @@ constexpr size_t sk_lds() {
 // F::a_off) and, for KIND 2, whose sub-block sums (bf16 hi[8] | lo[8]) start
 // at srow(t); then the block end of KIND 1 / 2 (the min term's two MFMAs
 // into acc, then acc += d * cb).  cb and cq are the block's own accumulators.
-// (GM, MERGE, PIN: as skinny_loop.)  OWN (KIND 3): the block's sub-blocks are
+// (GM, MERGE, PIN: as skinny_loop.)  OWN (KIND 3, and 4 at m <= 4): the block's sub-blocks are
 // summed apart and then added to acc, so a long K range is a sum of block sums
 // instead of one chain of 8 terms per block (Q8_0 at m = 2, k = 5120: error
 // against 64 bits 1.5e-7 -> 9.4e-8, the f32 GEMV's 9.8e-8; IQ4_XS, which has no
-// GEMV at m > 1 to match, ran 6 % longer with it).
+// GEMV at m > 1 to match, ran 6 % longer with it; Q6_K without it 4.1e-7 at one split
+// of k = 9216, 1.4e-7 with it, at 2 - 5 %: m <= 4 only, where the f32 GEMV was before).
 template <class F, int TA, int TU, int NW, int GM, bool MERGE, bool PIN, bool OWN = false, class XRow, class SRow>
 __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::Blk (&wbk)[NW], XRow xrow,
                                          SRow srow, int lr, int h, floatx16 (&acc)[NW][TA], floatx16 (&cb)[NW][TA],
@@ -466,11 +469,13 @@ __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::
     constexpr int KIND = F::KIND;
     constexpr int TO = MERGE ? TU / 2 : TU;  // accumulator tiles written
     constexpr int SL = F::RB + 16;           // slab row stride (bytes)
-    static_assert(!OWN || KIND == 3, "block sums apart: scaled per sub-block");
+    static_assert(!OWN || KIND >= 3, "block sums apart: scaled per sub-block");
     floatx16 own[OWN ? NW : 1][OWN ? TO : 1];
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-        if constexpr (PIN && TO == 2) __builtin_amdgcn_sched_barrier(0);
+        // (KIND 4 at f16 x and m <= 8: left free, 23 registers spilled, Q6_K 17408 -> 5120
+        // at m = 8 38.5 -> 23.9 us; where nothing spills the barrier costs 2 - 3 %)
+        if constexpr ((PIN && TO == 2) || (KIND == 4 && GM == 0x1)) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int w = 0; w < NW; w++) {
             half8 bf[4];
@@ -494,7 +499,15 @@ __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::
                     for (int ti = 0; ti < TO; ti++)
 #pragma unroll
                         for (int i = 0; i < 16; i++)
-                            if ((GM >> (4 * ti + (i >> 2))) & 1) acc[w][ti][i] = fmaf(ss, c[ti][i], acc[w][ti][i]);
+                            if ((GM >> (4 * ti + (i >> 2))) & 1) {
+                                if constexpr (OWN) {
+                                    own[w][ti][i] = p == 0 && kk == 0 ? ss * c[ti][i]
+                                                                      : fmaf(ss, c[ti][i], own[w][ti][i]);
+                                    if (p == 3 && kk == 3) acc[w][ti][i] += own[w][ti][i];
+                                } else {
+                                    acc[w][ti][i] = fmaf(ss, c[ti][i], acc[w][ti][i]);
+                                }
+                            }
                 } else {
 #pragma unroll
                     for (int t = 0; t < TU; t++) {
@@ -640,7 +653,10 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
             for (int i = 0; i < 8; i++) {
                 const float u = ldexpf(__uint_as_float(xv[i >> 2][i & 3]), xsh);
                 hp[0][i] = (_Float16)u;
-                const float r1 = u - (float)hp[0][i];  // exact
+                float r1 = u - (float)hp[0][i];  // exact
+                // an infinity is its own hi part, as the GEMVs of these formats multiply
+                // it (inf - inf would make every sum of the row NaN)
+                if constexpr (KIND != 2) r1 = (float)hp[0][i] == u ? 0.f : r1;
                 hp[1][i] = (_Float16)r1;
                 hp[2][i] = (_Float16)(r1 - (float)hp[1][i]);  // exact difference
             }
@@ -747,7 +763,8 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
         }
 #pragma unroll
         for (int o = 16; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));  // the row's 32 lanes
-        xsh = amax > 0.f && amax < INFINITY ? 15 - __builtin_amdgcn_frexp_expf(amax) : 0;
+        // (a row with an infinity: its finite elements stay below f16's largest)
+        xsh = amax == INFINITY ? 15 - 128 : amax > 0.f ? 15 - __builtin_amdgcn_frexp_expf(amax) : 0;
     }
     xload(b0);
     xstore(0);
@@ -770,7 +787,7 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
         // keep the scheduler from sinking the loads: they must be in flight
         // during this block, not issued at its end
         __builtin_amdgcn_sched_barrier(0);
-        sk_block<F, TA, TU, NW, GM, MERGE, PIN, XP == 3 && F::OWN>(
+        sk_block<F, TA, TU, NW, GM, MERGE, PIN, XP == 3 && F::OWN && (KIND == 3 || (GM & SK_OWN))>(
             slab, wb, [&](int t) { return xl + (xb * XR + 32 * t + lr) * SK_XLD; },
             [&](int t) { return sl + (xb * XR + 32 * t + lr) * 16; }, lr, h, acc, cb, cq);
 #pragma unroll

@@ -125,6 +125,31 @@ def test_m1_q8_0_infinite_x(gpu_ctx, oracle):
     w.free()
 
 
+@pytest.mark.parametrize("qtype,n,k,wide", [("q8_0", 4200, 3840, False), ("q6_k", 130, 4352, True),
+                                            ("q6_k", 130, 4352, False)])
+def test_small_m_infinite_x(gpu_ctx, oracle, qtype, n, k, wide):
+    # an infinite x in the skinny kernel's three-part form: +-inf in its own row, NaN
+    # (0 * inf) where its weight is 0, and the other rows as without it
+    _say("case: small m inf", qtype, n, k, wide)
+    m = 3
+    raw, x = synth.weight(qtype, n, k, seed=13), synth.activations(m, k, seed=14)
+    if wide:  # the form for scales over all of i8
+        rng = np.random.default_rng(n)
+        raw.reshape(-1, 210)[:, 192:208] = rng.integers(0, 256, size=(raw.size // 210, 16), dtype=np.uint8)
+    x[1, k - 3] = np.inf
+    w = gpu_ctx.upload(QType[qtype.upper()], raw, n, k)
+    y = gpu_ctx.empty((m, n), np.float32)
+    gpu_ctx.matmul(w, gpu_ctx.to_device(x), m, y)
+    got, wl = y.numpy(), oracle.dequant(qtype, raw, n * k).reshape(n, k)[:, k - 3]
+    with np.errstate(invalid="ignore"):
+        want = wl * np.float32(np.inf)
+    assert np.array_equal(np.isnan(got[1]), np.isnan(want))
+    fine = ~np.isnan(want)
+    assert np.array_equal(got[1][fine], want[fine])
+    assert _rel2(got[[0, 2]], _want(oracle, qtype, x[[0, 2]], raw, n)) <= 2.0 ** -20
+    w.free()
+
+
 @pytest.mark.parametrize("qg,qd,tokens,top_k,hidden,inter", [
     ("q4_k", "q6_k", 1, 2, 256, 512), ("q5_k", "q5_k", 3, 2, 768, 256), ("iq4_xs", "q6_k", 2, 3, 512, 1280),
     ("q8_0", "q8_0", 5, 1, 1280, 512), ("q6_k", "q4_k", 4, 2, 512, 768), ("iq4_xs", "iq4_xs", 1, 4, 4352, 256),
