@@ -448,11 +448,13 @@ template <class F, int TA, int PARTS, int GM = 0xFF, class XT = _Float16>
 static hipError_t launch_sk_t(const F &fmt, const arfq_weight *w, int64_t m, const XT *x,
                               const uint16_t *xs, const float *rs, int rss, float *y, float *part,
                               int S, hipStream_t s) {
+    if constexpr (std::is_base_of_v<SkQ6K, F> && PARTS == 3 && GM == 0xFF)
+        if (m <= 4)
+            return launch_sk_t<F, 1, 3, (F::KIND == 4 ? 0x7 : 0xFF) | SK_OWN, XT>(fmt, w, m, x, xs, rs, rss, y, part,
+                                                                               S, s);
     if constexpr (F::KIND >= 3 && TA == 1 && GM == 0xFF) {
         // at most 8 rows (8 hi + 8 lo with two parts, + 8 mid with three): the
         // per-sub-block scaling touches only the accumulator groups that hold them
-        if constexpr (F::KIND == 4 && PARTS == 3)
-            if (m <= 4) return launch_sk_t<F, 1, 3, 0x7 | SK_OWN, XT>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
         if (m <= 8)
             return launch_sk_t<F, 1, PARTS, PARTS == 3 ? 0x7 : PARTS == 2 ? 0x5 : 0x1, XT>(fmt, w, m, x, xs, rs, rss,
                                                                                           y, part, S, s);

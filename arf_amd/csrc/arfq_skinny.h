@@ -430,7 +430,8 @@ struct SkRows {
     int64_t s;      // element offset (row * K / 16) of row min(tid >> 1, XR - 1)
 };
 
-constexpr int SK_OWN = 0x100;  // a bit of GM: KIND 4 sums each block apart
+// a bit of GM (Q6_K at m <= 4): an infinite x stays one, and KIND 4 sums each block apart
+constexpr int SK_OWN = 0x100;
 
 // Where 16-byte unit u of a weight row's block lies in the row's slab: as it comes, but
 // for Q6_K's chunks.
@@ -655,8 +656,9 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
                 hp[0][i] = (_Float16)u;
                 float r1 = u - (float)hp[0][i];  // exact
                 // an infinity is its own hi part, as the GEMVs of these formats multiply
-                // it (inf - inf would make every sum of the row NaN)
-                if constexpr (KIND != 2) r1 = (float)hp[0][i] == u ? 0.f : r1;
+                // it (inf - inf would make every sum of the row NaN); Q6_K only at m <= 4,
+                // which had a GEMV: at m = 8 the compare took 28.6 -> 29.1 us
+                if constexpr (KIND == 3 ? F::OWN : (GM & SK_OWN) != 0) r1 = (float)hp[0][i] == u ? 0.f : r1;
                 hp[1][i] = (_Float16)r1;
                 hp[2][i] = (_Float16)(r1 - (float)hp[1][i]);  // exact difference
             }
