@@ -1034,8 +1034,10 @@ struct DotQ6K {
         return A * (xsc * (float)sdot - 32.f * xsum);
     }
     // the f32-x kernel's codes are the bytes xor FXOR (unsigned), its quadrant
-    // term; its xsum arrives as XSUM_MUL * sum(x), scaled where x is read from LDS
+    // term; its xsum arrives as XSUM_MUL * sum(x), scaled where x is read from LDS.
+    // BIAS > 0: the bytes are BIAS above the signed codes
     static constexpr uint32_t FXOR = 0u;
+    static constexpr int BIAS = 32;
     static constexpr float XSUM_MUL = -32.f;
     static constexpr bool SIGNED = false;
     __device__ static float fterm(float A, float B, float xsc, float dot, float xsum) {
@@ -1125,6 +1127,7 @@ struct DotQ5K {
         return A * (xsc * (float)sdot) - B * xsum;
     }
     static constexpr uint32_t FXOR = 0u;
+    static constexpr int BIAS = 0;
     static constexpr float XSUM_MUL = 1.f;
     static constexpr bool SIGNED = false;
     __device__ static float fterm(float A, float B, float xsc, float dot, float xsum) {
@@ -1210,6 +1213,7 @@ struct DotIQ4XS {
     }
     // f32 x: the unsigned codes kv + 128 (kv xor 0x80), less 128 * sum(x)
     static constexpr uint32_t FXOR = 0x80808080u;
+    static constexpr int BIAS = 128;
     static constexpr float XSUM_MUL = -128.f;
     static constexpr bool SIGNED = false;
     __device__ static float fterm(float A, float B, float xsc, float dot, float xsum) {
@@ -1268,6 +1272,7 @@ struct DotQ80 {
         for (int j = 0; j < 4; j++) cw[j] = l.q[t][j];
     }
     static constexpr uint32_t FXOR = 0u;
+    static constexpr int BIAS = 0;
     static constexpr float XSUM_MUL = 0.f;
     static constexpr bool SIGNED = true;
     __device__ static float fterm(float A, float, float xsc, float dot, float) { return A * (xsc * dot); }
@@ -1437,7 +1442,8 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot(F fmt, const float 
 // weight (gguf.rs:2120-2123) times f32 x, factorised.
 namespace {
 
-__device__ __forceinline__ void xf16_process(const XqRound &r, int items, int base, float4 *xf,
+// (returns whether the sum of the thread's 16 elements, times a code, may not be finite)
+__device__ __forceinline__ bool xf16_process(const XqRound &r, int items, int base, float4 *xf,
                                              float *s16, float *xe) {
     const int it = base + (int)threadIdx.x;
     const float4 v0 = r.v0, v1 = r.v1;
@@ -1447,7 +1453,8 @@ __device__ __forceinline__ void xf16_process(const XqRound &r, int items, int ba
     amax = fmaxf(amax, quad_perm<QP_XOR1>(amax));
     sum += quad_perm<QP_XOR1>(sum);  // 16 elements (items 2i, 2i + 1)
     amax = fmaxf(amax, quad_perm<QP_XOR2>(amax));
-    const int ex = (amax > 0.f) ? __builtin_amdgcn_frexp_expf(amax) : 0;
+    // (beside an infinity, whose exponent reads as 0, the finite elements must not overflow)
+    const int ex = amax == INFINITY ? 128 : (amax > 0.f) ? __builtin_amdgcn_frexp_expf(amax) : 0;
     const int sh = min(24, 100 - ex);
     if (it < items) {
         xf[2 * it] = make_float4(ldexpf(v0.x, sh), ldexpf(v0.y, sh), ldexpf(v0.z, sh), ldexpf(v0.w, sh));
@@ -1455,6 +1462,7 @@ __device__ __forceinline__ void xf16_process(const XqRound &r, int items, int ba
         if ((it & 1) == 0) s16[it >> 1] = sum;
         if ((it & 3) == 0) xe[it >> 2] = ldexpf(1.f, 24 - sh);
     }
+    return !(fabsf(sum) * 256.f < INFINITY);
 }
 
 // sum of x * q over 16 codes (one byte each in cw[4], element order), x scaled
@@ -1473,20 +1481,50 @@ __device__ __forceinline__ float codes16_fdot(const uint32_t cw[4], const float 
     return acc;
 }
 
+// the same with the bytes less BIAS: put under 0x64 (the f16 1024 + byte) and reduced
+// to the signed code, exact; the codes are whole, not q * 2^-24
+template <int BIAS>
+__device__ __forceinline__ float codes16_sdot(const uint32_t cw[4], const float *X) {
+    const f16x2v off = {(_Float16)(-1024 - BIAS), (_Float16)(-1024 - BIAS)};
+    auto code = [&](uint32_t w, uint32_t sel) {
+        return __builtin_bit_cast(uint32_t,
+                                  __builtin_bit_cast(f16x2v, __builtin_amdgcn_perm(0x64646464u, w, sel)) + off);
+    };
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t A = code(cw[j], 0x04020400u), B = code(cw[j], 0x04030401u);
+        acc = fmix<0>(X[4 * j], A, acc);
+        acc = fmix<1>(X[4 * j + 2], A, acc);
+        acc = fmix<0>(X[4 * j + 1], B, acc);
+        acc = fmix<1>(X[4 * j + 3], B, acc);
+    }
+    return acc;
+}
+
 }  // namespace
 
 // Rows: workgroup w of G owns rows w, w + G, w + 2G, ... (the whole chip reads a
 // narrow window of the weight stream at a time), and x is scaled into LDS
 // before the first weight load is issued (every weight request in flight
 // delays the x requests); as the Q4_K f32 GEMV (gemv_q4k_f32_body).
+// Formats with a BIAS: an x whose sum over some quadrant is not finite (the bytes less
+// BIAS * sum(x) would be inf - inf for every code) has its rows done again at the end
+// with the signed codes.  IQ4_XS takes those for every f16 x (SG: 16.1 -> 18.1 us at
+// 17408 x 5120, but error against 64 bits 1.04e-7 -> 7.5e-8 at 4096 x 1024; the skinny
+// kernel, without a bias to cancel, has 8.2e-8.  At f32 x the bytes' 2.0e-7 would be
+// 1.0e-7, for 11 % more time, 6 % for Q6_K; a branch on x in the loop took 28
+// registers).
 template <class F, int XR, class XSRC>
 __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc, float *__restrict__ y, int n,
                                                   int nblk) {
+    constexpr bool SG = F::BIAS == 128 && std::is_same_v<XSRC, XsF16>;
     constexpr int C = Q6K_GEMV_CHUNK, PF = F::PF;
     static_assert(PF % C == 0, "claims must sit at fixed slots of the unrolled loop");
     extern __shared__ uint4 smem4[];
     __shared__ int cnt[64];             // chunk counters per column (spr <= 64)
     __shared__ unsigned long long exm;  // columns seen exhausted
+    __shared__ int redo;                // some sum(x) is not finite
     const int k = nblk * 256;
     float *xfl = reinterpret_cast<float *>(smem4);  // [k], scaled
     float *s16 = xfl + k;                           // [k / 16]
@@ -1573,7 +1611,7 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
 
     // counters start past the chunks the groups begin on
     for (int cc = tid; cc < spr; cc += Q6K_GEMV_THREADS) cnt[cc] = (Q6K_GEMV_GROUPS - cc + spr - 1) / spr;
-    if (tid == 0) exm = 0;
+    if (tid == 0) exm = 0, redo = 0;
     // x loads, x scaled into LDS, the barrier (which orders LDS only), then the
     // first weight loads
     const int xitems = k / 8;
@@ -1581,12 +1619,14 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
 #pragma unroll
     for (int r = 0; r < XR; r++) xr[r] = xsrc.load(xitems, r * Q6K_GEMV_THREADS);
     asm volatile("" ::: "memory");
+    bool odd = false;
 #pragma unroll
     for (int r = 0; r < XR; r++)
-        xf16_process(xr[r], xitems, r * Q6K_GEMV_THREADS, reinterpret_cast<float4 *>(xfl), s16, xe);
+        odd |= xf16_process(xr[r], xitems, r * Q6K_GEMV_THREADS, reinterpret_cast<float4 *>(xfl), s16, xe);
     for (int base = XR * Q6K_GEMV_THREADS; base < xitems; base += Q6K_GEMV_THREADS)
-        xf16_process(xsrc.load(xitems, base), xitems, base, reinterpret_cast<float4 *>(xfl), s16, xe);
+        odd |= xf16_process(xsrc.load(xitems, base), xitems, base, reinterpret_cast<float4 *>(xfl), s16, xe);
     lds_barrier();
+    if (F::BIAS != 0 && !SG && odd) redo = 1;  // read past the next barrier
 #pragma unroll
     for (int u = 0; u < PF; u++) issue(u, u < C);
 
@@ -1598,9 +1638,9 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
         const int xb = F::COLUMN ? F::xbase(col, l16) : F::xbase(min(4 * col + bq, nblk - 1), c);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            // (COLUMN: a block past the row has zero codes, and takes x = 0)
-            const bool in = !F::COLUMN || 4 * col + t < nblk;
-            const int eo = in ? xb + F::xoff(t) : 0;
+            // (a block past the row has zero bytes; signed codes take x = 0 with it)
+            const bool in = 4 * col + (F::COLUMN ? t : bq) < nblk;
+            const int eo = in || !F::COLUMN ? xb + F::xoff(t) : 0;
             const float4 *src = reinterpret_cast<const float4 *>(xfl + eo);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -1610,12 +1650,12 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
                 X[t][4 * i + 2] = v.z;
                 X[t][4 * i + 3] = v.w;
             }
-            if constexpr (F::COLUMN) {
+            if constexpr (F::COLUMN || SG) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) X[t][i] = in ? X[t][i] : 0.f;
             }
             XS[t] = F::XSUM_MUL * s16[eo >> 4];
-            XE[t] = xe[eo >> 5];
+            XE[t] = (SG ? 0x1p-24f : 1.f) * xe[eo >> 5];
         }
     };
 
@@ -1631,8 +1671,13 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
         for (int t = 0; t < 4; t++) {
             uint32_t cw[4];
             F::template codes<F::FXOR>(ld[u], c, t, cw);
-            const float dot = F::SIGNED ? dot16_i8(X[t], make_uint4(cw[0], cw[1], cw[2], cw[3])) : codes16_fdot(cw, X[t]);
-            v += F::fterm(A[t], B[t], XE[t], dot, XS[t]);
+            if constexpr (SG) {
+                v += A[t] * (XE[t] * codes16_sdot<F::BIAS>(cw, X[t]));
+            } else {
+                const float dot =
+                    F::SIGNED ? dot16_i8(X[t], make_uint4(cw[0], cw[1], cw[2], cw[3])) : codes16_fdot(cw, X[t]);
+                v += F::fterm(A[t], B[t], XE[t], dot, XS[t]);
+            }
         }
         v = row16_sum(v);
         if (l16 == 0 && live) part[(size_t)row * spr + col] = v;
@@ -1647,11 +1692,36 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
     }
     lds_barrier();
 
+    const bool again = F::BIAS != 0 && !SG && redo;  // (read with the sums: no wait of its own)
     for (int t = tid; t < R; t += Q6K_GEMV_THREADS) {
         const float *pr = part + (size_t)t * spr;
         float v = 0.f;
         for (int cc = 0; cc < spr; cc++) v += pr[cc];
-        y[r0 + t * G] = v;
+        if (__builtin_expect(!again, 1)) y[r0 + t * G] = v;
+    }
+    if constexpr (F::BIAS != 0 && !SG) {
+        if (__builtin_expect(again, 0)) {  // a 16-lane group per row
+            for (int row = grp; row < R; row += Q6K_GEMV_GROUPS) {
+                float v = 0.f;
+#pragma unroll 1
+                for (int b = bq; b < 4 * spr; b += 4) {
+                    typename F::Lane l;
+                    F::load(res, l, (uint32_t)(r0 + row * G) * (uint32_t)nblk + (uint32_t)b, b < nblk, c);
+                    F::expand(l);
+                    float A[4], B[4];
+                    F::scales(l, c, A, B);
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        uint32_t cw[4];
+                        F::template codes<F::FXOR>(l, c, t, cw);
+                        const int eo = F::xbase(b, c) + F::xoff(t);
+                        if (b < nblk) v += A[t] * (0x1p-24f * xe[eo >> 5] * codes16_sdot<F::BIAS>(cw, xfl + eo));
+                    }
+                }
+                v = row16_sum(v);
+                if (l16 == 0) y[r0 + row * G] = v;
+            }
+        }
     }
 }
 

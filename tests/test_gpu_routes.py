@@ -125,6 +125,50 @@ def test_m1_q8_0_infinite_x(gpu_ctx, oracle):
     w.free()
 
 
+@pytest.mark.parametrize("qtype,n,k", [("q6_k", 130, 256), ("q6_k", 700, 4352), ("iq4_xs", 1030, 1792),
+                                       ("iq4_xs", 3, 8448), ("q8_0", 13000, 1280)])
+@pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("at", [0, -3])
+def test_m1_infinite_x(gpu_ctx, oracle, qtype, n, k, x_dtype, at):
+    # +-inf by the sign of its weight, NaN (0 * inf) where that is 0, in one x row of f32 or
+    # f16: the first block, or a last column of one or three blocks
+    _say("case: m1 inf", qtype, n, k, np.dtype(x_dtype).name, at)
+    raw, x = synth.weight(qtype, n, k, seed=21), synth.activations(1, k, seed=22).astype(x_dtype)
+    x[0, at] = -np.inf
+    if x_dtype == np.float32:
+        x[0, at ^ 1] = 3e38  # finite: beside the infinity it changes nothing
+    w = gpu_ctx.upload(QType[qtype.upper()], raw, n, k)
+    y = gpu_ctx.empty((1, n), np.float32)
+    gpu_ctx.matmul(w, gpu_ctx.to_device(x), 1, y)
+    with np.errstate(invalid="ignore"):
+        want = oracle.dequant(qtype, raw, n * k).reshape(n, k)[:, at] * np.float32(-np.inf)
+    assert np.array_equal(y.numpy()[0], want, equal_nan=True)
+    w.free()
+
+
+@pytest.mark.parametrize("qd", ["q6_k", "iq4_xs", "q8_0"])
+def test_moe_pairs_infinite_h(gpu_ctx, oracle, qd):
+    # one row of gate and up is not 0, and its g and u overflow h = silu(g) * u to inf: y is
+    # +-inf by the sign of down's column of that row
+    _say("case: moe inf", qd)
+    E, hidden, inter, j = 2, 512, 1280, 1277
+    gu = synth.weight("q8_0", inter, hidden, seed=31, experts=E).reshape(E, inter, hidden // 32, 34)
+    gu[:, :, :, :2] = 0
+    gu[:, j, :, 1] = 0x3C  # d = 1 in row j
+    gu[:, j, :, 2:] = 1
+    dn = synth.weight(qd, hidden, inter, seed=32, experts=E)
+    ws = [gpu_ctx.upload(QType.Q8_0, gu.reshape(-1), inter, hidden, E) for _ in range(2)]
+    ws.append(gpu_ctx.upload(QType[qd.upper()], dn, hidden, inter, E))
+    ids, wts = np.array([[1]], np.int32), np.ones((1, 1), np.float32)
+    x, y = np.full((1, hidden), 1e25, np.float32), gpu_ctx.empty((1, hidden), np.float32)
+    gpu_ctx.moe_ids(*ws, gpu_ctx.to_device(ids), gpu_ctx.to_device(wts), 1, 1, gpu_ctx.to_device(x), y)
+    with np.errstate(invalid="ignore"):
+        want = oracle.dequant(qd, dn, E * hidden * inter).reshape(E, hidden, inter)[1, :, j] * np.float32(np.inf)
+    assert np.array_equal(y.numpy()[0], want, equal_nan=True)
+    for w in ws:
+        w.free()
+
+
 @pytest.mark.parametrize("qtype,n,k,wide", [("q8_0", 4200, 3840, False), ("q6_k", 130, 4352, True),
                                             ("q6_k", 130, 4352, False)])
 def test_small_m_infinite_x(gpu_ctx, oracle, qtype, n, k, wide):
