@@ -448,17 +448,6 @@ template <class F, int TA, int PARTS, int GM = 0xFF, class XT = _Float16>
 static hipError_t launch_sk_t(const F &fmt, const arfq_weight *w, int64_t m, const XT *x,
                               const uint16_t *xs, const float *rs, int rss, float *y, float *part,
                               int S, hipStream_t s) {
-    if constexpr (std::is_base_of_v<SkQ6K, F> && PARTS == 3 && GM == 0xFF)
-        if (m <= 4)
-            return launch_sk_t<F, 1, 3, (F::KIND == 4 ? 0x7 : 0xFF) | SK_OWN, XT>(fmt, w, m, x, xs, rs, rss, y, part,
-                                                                               S, s);
-    if constexpr (F::KIND >= 3 && TA == 1 && GM == 0xFF) {
-        // at most 8 rows (8 hi + 8 lo with two parts, + 8 mid with three): the
-        // per-sub-block scaling touches only the accumulator groups that hold them
-        if (m <= 8)
-            return launch_sk_t<F, 1, PARTS, PARTS == 3 ? 0x7 : PARTS == 2 ? 0x5 : 0x1, XT>(fmt, w, m, x, xs, rs, rss,
-                                                                                          y, part, S, s);
-    }
     constexpr int NT = sk_nt(TA), CT = NT / 2;
     constexpr size_t lds = sk_lds<F, TA, 1, NT, SK_XB(TA)>() + 32 * TA * 4;  // + the x rows' scales
     static std::atomic<uint64_t> lds_set{0};  // the attribute belongs to the kernel, per device
@@ -479,7 +468,18 @@ static hipError_t launch_sk_t(const F &fmt, const arfq_weight *w, int64_t m, con
     return hipSuccess;
 }
 
-// S > 1 splits need S <= 16 and one zeroed counter per column tile.  x is
+// At most 8 rows, as one f16 part or three parts (8 hi + 8 mid + 8 lo): the per-sub-block
+// scaling of KIND 3 and 4 touches only the accumulator groups that hold them.
+template <class F, int PARTS, class XT>
+static hipError_t launch_sk_m8(const F &fmt, const arfq_weight *w, int64_t m, const XT *x, const uint16_t *xs,
+                               const float *rs, int rss, float *y, float *part, int S, hipStream_t s) {
+    constexpr int GM = F::KIND < 3 ? 0xFF : PARTS == 3 ? 0x7 : 0x1;
+    if constexpr (std::is_base_of_v<SkQ6K, F> && PARTS == 3)
+        if (m <= 4) return launch_sk_t<F, 1, 3, GM | SK_OWN, XT>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
+    return launch_sk_t<F, 1, PARTS, GM, XT>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
+}
+
+// S > 1 splits need S <= 16 and their partials' scratch.  x is
 // f16 (an f32 x arrives prepared and scaled, rs[split * rss + row] its scale
 // over each split's K range); with parts 2 (m <= 64) it is [2m, K]: the hi
 // rows, then the lo rows; with parts 3 (m <= 8) the caller's f32 x [m, K] as
@@ -493,7 +493,7 @@ static hipError_t launch_sk(const F &fmt, const arfq_weight *w, int64_t m, const
     if (parts == 3) {
         if (m > 8) return hipErrorInvalidValue;
         if (!xf) return hipErrorInvalidValue;
-        return launch_sk_t<F, 1, 3, 0xFF, float>(fmt, w, m, xf, nullptr, nullptr, 0, y, part, S, s);
+        return launch_sk_m8<F, 3, float>(fmt, w, m, xf, nullptr, nullptr, 0, y, part, S, s);
     }
     if (parts == 2) {
         if (m > 64) return hipErrorInvalidValue;
@@ -501,6 +501,7 @@ static hipError_t launch_sk(const F &fmt, const arfq_weight *w, int64_t m, const
         if (m <= 32) return launch_sk_t<F, 2, 2>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
         return launch_sk_t<F, 4, 2>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
     }
+    if (m <= 8) return launch_sk_m8<F, 1, _Float16>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
     return m <= 32 ? launch_sk_t<F, 1, 1>(fmt, w, m, x, xs, rs, rss, y, part, S, s)
                    : launch_sk_t<F, 2, 1>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
 }
