@@ -150,14 +150,17 @@ struct SkQ6K {
     __device__ const uint8_t *raw(int64_t row, int b) const {
         return reinterpret_cast<const uint8_t *>(qb8 + (row * nblk + b) * 24);
     }
-    // The slab holds the block as chunks of 48 bytes, ql_a | ql_b | qh: 16-byte unit u
-    // of the stream (see q6k_off) goes to unit slab_unit(u).  (In the stream's own
-    // order the reads of two steps look alike to the compiler, which merges them and
-    // holds both steps' bytes: the kernel of m = 17..32 spilled and a product there took
-    // 302 us instead of 199.)
-    __device__ static int slab_unit(int u) {
-        const int n2 = u >= 6, v = u - 6 * n2;
-        return 6 * n2 + 3 * (v & 1) + (v >> 1);
+    // Chunk p's ql_a bytes of lane half h in the slab row.  APART: the offset goes through
+    // an empty asm.  Without it the compiler reads the chunks of two steps, 16 bytes apart,
+    // together and holds both steps' bytes (the kernel of m = 17..32 spilled, a product
+    // there took 302 us instead of 199).  Where nothing spills it costs (f32 x at m = 4,
+    // 17408 -> 5120: 27.4 us without, 28.7 with).  A slab of 48-byte chunks kept the steps
+    // apart too, but its permuted stores took 1 % (m = 8 28.8 us against 28.4).
+    template <bool APART>
+    __device__ static const uint8_t *chunk(const uint8_t *srow, int p, int h) {
+        int o = q6k_off(p) + 8 * h;
+        if constexpr (APART) asm("" : "+v"(o));
+        return srow + o;
     }
     __device__ Blk load_blk(int64_t row, int b) const {
         return {ldv(sc16 + row * nblk + b), dd[row * nblk + b]};
@@ -183,11 +186,12 @@ struct SkQ6K {
     }
     // q - 32: v_perm puts two code bytes under 0x64 (the f16 1024 + q), less
     // 1056, exact
+    template <bool APART>
     __device__ static void frag(const uint8_t *srow, const Blk &, int p, int h, half8 f[4]) {
-        const uint8_t *ch = srow + 48 * p;
-        const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch + 8 * h);
-        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + 16 + 8 * h);
-        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + 32 + 8 * h);
+        const uint8_t *ch = chunk<APART>(srow, p, h);
+        const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch);
+        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + Q6K_QB);
+        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + Q6K_QH);
         const half2v m1056 = h2splat(-1056.f);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -219,11 +223,12 @@ struct SkQ6KI : SkQ6K {
     static constexpr bool OWN = false;
     __host__ __device__ SkQ6KI shifted(int64_t nb) const { return {SkQ6K::shifted(nb)}; }
     __device__ static float2 scale(const Blk &k) { return make_float2(2.f * h2f(k.d), 0.f); }
+    template <bool APART>
     __device__ static void frag(const uint8_t *srow, const Blk &k, int p, int h, half8 f[4]) {
-        const uint8_t *ch = srow + 48 * p;
-        const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch + 8 * h);
-        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + 16 + 8 * h);
-        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + 32 + 8 * h);
+        const uint8_t *ch = chunk<APART>(srow, p, h);
+        const u32x2 qa = *reinterpret_cast<const u32x2 *>(ch);
+        const u32x2 qb = *reinterpret_cast<const u32x2 *>(ch + Q6K_QB);
+        const u32x2 qh = *reinterpret_cast<const u32x2 *>(ch + Q6K_QH);
         // scale bytes as sc + 128 (unsigned)
         const uint32_t scw[4] = {k.sc.x ^ 0x80808080u, k.sc.y ^ 0x80808080u, k.sc.z ^ 0x80808080u,
                                  k.sc.w ^ 0x80808080u};
@@ -433,16 +438,6 @@ struct SkRows {
 // a bit of GM (Q6_K at m <= 4): an infinite x stays one, and KIND 4 sums each block apart
 constexpr int SK_OWN = 0x100;
 
-// Where 16-byte unit u of a weight row's block lies in the row's slab: as it comes, but
-// for Q6_K's chunks.
-template <class F>
-__device__ __forceinline__ int slab_unit(int u) {
-    if constexpr (std::is_base_of_v<SkQ6K, F>)
-        return F::slab_unit(u);
-    else
-        return u;
-}
-
 // LDS of the loop: XB buffers of the x block of XR rows (+ its sub-block sums)
 // and one weight slab [32][RB + 16] per wave and weight.
 template <class F, int TA, int NW, int NT = SK_THREADS, int XB = 1>
@@ -463,7 +458,9 @@ constexpr size_t sk_lds() {
 // against 64 bits 1.5e-7 -> 9.4e-8, the f32 GEMV's 9.8e-8; IQ4_XS, which has no
 // GEMV at m > 1 to match, ran 6 % longer with it; Q6_K without it 4.1e-7 at one split
 // of k = 9216, 1.4e-7 with it, at 2 - 5 %: m <= 4 only, where the f32 GEMV was before).
-template <class F, int TA, int TU, int NW, int GM, bool MERGE, bool PIN, bool OWN = false, class XRow, class SRow>
+// APART (Q6_K): SkQ6K::chunk.
+template <class F, int TA, int TU, int NW, int GM, bool MERGE, bool PIN, bool OWN = false, bool APART = true,
+          class XRow, class SRow>
 __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::Blk (&wbk)[NW], XRow xrow,
                                          SRow srow, int lr, int h, floatx16 (&acc)[NW][TA], floatx16 (&cb)[NW][TA],
                                          floatx16 (&cq)[NW][F::KIND == 3 ? TA : 1]) {
@@ -480,7 +477,10 @@ __device__ __forceinline__ void sk_block(const uint8_t *slab, const typename F::
 #pragma unroll
         for (int w = 0; w < NW; w++) {
             half8 bf[4];
-            F::frag(slab + (w * 32 + lr) * SL, wbk[w], p, h, bf);
+            if constexpr (std::is_base_of_v<SkQ6K, F>)
+                F::template frag<APART>(slab + (w * 32 + lr) * SL, wbk[w], p, h, bf);
+            else
+                F::frag(slab + (w * 32 + lr) * SL, wbk[w], p, h, bf);
 #pragma unroll
             for (int kk = 0; kk < 4; kk++) {
                 if constexpr (KIND == 4) {
@@ -732,7 +732,7 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
 #pragma unroll
             for (int i = 0; i < NI; i++) {
                 const int c = 64 * i + lane;
-                *reinterpret_cast<u32x4 *>(slab + (w * 32 + c / RL) * SL + 16 * slab_unit<F>(c % RL)) = rv[w][i];
+                *reinterpret_cast<u32x4 *>(slab + (w * 32 + c / RL) * SL + 16 * (c % RL)) = rv[w][i];
             }
     };
     int64_t myrow[NW];
@@ -789,7 +789,7 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
         // keep the scheduler from sinking the loads: they must be in flight
         // during this block, not issued at its end
         __builtin_amdgcn_sched_barrier(0);
-        sk_block<F, TA, TU, NW, GM, MERGE, PIN, XP == 3 && F::OWN && (KIND == 3 || (GM & SK_OWN))>(
+        sk_block<F, TA, TU, NW, GM, MERGE, PIN, XP == 3 && F::OWN && (KIND == 3 || (GM & SK_OWN)), XP != 3>(
             slab, wb, [&](int t) { return xl + (xb * XR + 32 * t + lr) * SK_XLD; },
             [&](int t) { return sl + (xb * XR + 32 * t + lr) * 16; }, lr, h, acc, cb, cq);
 #pragma unroll
