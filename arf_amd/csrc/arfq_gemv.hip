@@ -2322,19 +2322,23 @@ bool gemv_pairs_supports(const arfq_weight *w, int64_t P, int nz) {
 
 // The dot formats' pairs: y0 row p = W0_ids[p] . x_p and, with w1 (same qtype and
 // shape), y1 row p = W1_ids[p] . x_p in the same launch.
+template <class F, int XR, class XS>
+static hipError_t launch_dot_pairs_t(const F &f0, const F &f1, const arfq_weight *w, int nz, int64_t P,
+                                     const int32_t *ids, const XS &xs, float *y0, float *y1, hipStream_t s) {
+    static std::atomic<uint64_t> lds_set{0};  // the attribute belongs to the kernel, per device
+    if (hipError_t err = set_max_lds_once((const void *)gemv_dot_pairs<F, XR, XS>, DOT_F32_LDS_MAX, lds_set))
+        return err;
+    const int64_t g = pairs_grid(w, P, nz);
+    gemv_dot_pairs<F, XR, XS>
+        <<<dim3((unsigned)g, (unsigned)P, (unsigned)nz), Q6K_GEMV_THREADS, dot_pairs_lds(w, g), s>>>(
+            f0, f1, xs, y0, y1, (int)w->n, (int)(w->k / 256), ids, w->experts);
+    return hipGetLastError();
+}
 template <class F, class XS>
 static hipError_t launch_dot_pairs_f(const F &f0, const F &f1, const arfq_weight *w, int nz, int64_t P,
                                      const int32_t *ids, const XS &xs, float *y0, float *y1, hipStream_t s) {
-    const int64_t g = pairs_grid(w, P, nz);
-    const dim3 grid((unsigned)g, (unsigned)P, (unsigned)nz);
-    const size_t lds = dot_pairs_lds(w, g);
-    auto go = [&](auto kern) -> hipError_t {
-        static std::atomic<uint64_t> lds_set{0};
-        if (hipError_t err = set_max_lds_once((const void *)kern, DOT_F32_LDS_MAX, lds_set)) return err;
-        kern<<<grid, Q6K_GEMV_THREADS, lds, s>>>(f0, f1, xs, y0, y1, (int)w->n, (int)(w->k / 256), ids, w->experts);
-        return hipGetLastError();
-    };
-    return w->k <= Q6K_GEMV_THREADS * 8 ? go(gemv_dot_pairs<F, 1, XS>) : go(gemv_dot_pairs<F, 2, XS>);
+    if (w->k <= Q6K_GEMV_THREADS * 8) return launch_dot_pairs_t<F, 1>(f0, f1, w, nz, P, ids, xs, y0, y1, s);
+    return launch_dot_pairs_t<F, 2>(f0, f1, w, nz, P, ids, xs, y0, y1, s);
 }
 template <class XS>
 static hipError_t launch_dot_pairs(const arfq_weight *w0, const arfq_weight *w1, int64_t P, const int32_t *ids,
@@ -2431,25 +2435,24 @@ hipError_t launch_gemv_glu(const arfq_weight *w, int64_t m, const float *g, cons
     return hipErrorInvalidValue;
 }
 
+template <int XR, class XS>
+static hipError_t launch_q4k_pairs_dual_t(const arfq_weight *w0, const arfq_weight *w1, int64_t P,
+                                          const int32_t *ids, const XS &xs, float *y0, float *y1, hipStream_t s) {
+    static std::atomic<uint64_t> lds_set{0};  // the attribute belongs to the kernel, per device
+    if (hipError_t err = set_max_lds_once((const void *)gemv_q4k_pairs_dual<XR, XS>, Q4K_F32_LDS_MAX, lds_set))
+        return err;
+    const int64_t g = pairs_grid(w0, P, 2), nb = w0->n * (w0->k / 256);
+    gemv_q4k_pairs_dual<XR, XS><<<dim3((unsigned)g, (unsigned)P, 2), Q4K_GEMV_THREADS, q4k_pairs_lds(w0, g), s>>>(
+        (const uint8_t *)w0->s0, (const uint8_t *)w0->s1, (const uint8_t *)w1->s0, (const uint8_t *)w1->s1,
+        (uint32_t)(nb * 16), (uint32_t)(nb * 128), xs, y0, y1, (int)w0->n, (int)(w0->k / 256), ids, w0->experts);
+    return hipGetLastError();
+}
 template <class XS>
 static hipError_t launch_pairs_dual_t(const arfq_weight *w0, const arfq_weight *w1, int64_t P,
                                       const int32_t *ids, const XS &xs, float *y0, float *y1, hipStream_t s) {
     if (w0->qtype != ARFQ_Q4_K) return launch_dot_pairs(w0, w1, P, ids, xs, y0, y1, s);
-    const int64_t g = pairs_grid(w0, P, 2);
-    const int64_t nb = w0->n * (w0->k / 256);
-    const dim3 grid((unsigned)g, (unsigned)P, 2);
-    const size_t lds = q4k_pairs_lds(w0, g);
-    auto go = [&](auto kern) -> hipError_t {
-        static std::atomic<uint64_t> lds_set{0};
-        if (hipError_t err = set_max_lds_once((const void *)kern, Q4K_F32_LDS_MAX, lds_set)) return err;
-        kern<<<grid, Q4K_GEMV_THREADS, lds, s>>>((const uint8_t *)w0->s0, (const uint8_t *)w0->s1,
-                                                 (const uint8_t *)w1->s0, (const uint8_t *)w1->s1,
-                                                 (uint32_t)(nb * 16), (uint32_t)(nb * 128), xs, y0, y1,
-                                                 (int)w0->n, (int)(w0->k / 256), ids, w0->experts);
-        return hipGetLastError();
-    };
-    if ((int)(w0->k / 32) * 4 <= Q4K_GEMV_THREADS) return go(gemv_q4k_pairs_dual<1, XS>);
-    return go(gemv_q4k_pairs_dual<2, XS>);
+    if (w0->k / 32 * 4 <= Q4K_GEMV_THREADS) return launch_q4k_pairs_dual_t<1>(w0, w1, P, ids, xs, y0, y1, s);
+    return launch_q4k_pairs_dual_t<2>(w0, w1, P, ids, xs, y0, y1, s);
 }
 
 bool gemv_pairs_dual_supports(const arfq_weight *w0, const arfq_weight *w1, int64_t P) {

@@ -194,17 +194,8 @@ def test_small_m_infinite_x(gpu_ctx, oracle, qtype, n, k, wide):
     w.free()
 
 
-@pytest.mark.parametrize("qg,qd,tokens,top_k,hidden,inter", [
-    ("q4_k", "q6_k", 1, 2, 256, 512), ("q5_k", "q5_k", 3, 2, 768, 256), ("iq4_xs", "q6_k", 2, 3, 512, 1280),
-    ("q8_0", "q8_0", 5, 1, 1280, 512), ("q6_k", "q4_k", 4, 2, 512, 768), ("iq4_xs", "iq4_xs", 1, 4, 4352, 256),
-    ("q5_k", "q6_k", 70, 2, 512, 512), ("q8_0", "iq4_xs", 66, 2, 256, 256)])
-@pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
-def test_moe_pairs_and_grouped(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, inter, x_dtype):
-    # up to 128 pairs: the f32 GEMVs (each product's sums below 2^-20, g and u through
-    # silu(g) * u and the down sums: four such errors, 2^-18).  More pairs: the grouped
-    # kernels, x and h in f16 (2^-11 each).  One id of the given ones is out of range and
-    # adds nothing.
-    _say("case: moe", qg, qd, tokens, top_k, hidden, inter, np.dtype(x_dtype).name)
+def _moe(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, inter, x_dtype):
+    """moe_ids over four experts, the last id out of range, and the same in float64."""
     E = 4
     shapes = [(qg, inter, hidden), (qg, inter, hidden), (qd, hidden, inter)]
     raw = [synth.weight(q, n, k, seed=50 + i, experts=E) for i, (q, n, k) in enumerate(shapes)]
@@ -224,7 +215,32 @@ def test_moe_pairs_and_grouped(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, i
                 g, u = dq[0][e] @ x[t].astype(np.float64), dq[1][e] @ x[t].astype(np.float64)
                 with np.errstate(over="ignore"):
                     want[t] += wt * (dq[2][e] @ (g / (1 + np.exp(-g)) * u))
-    got = y.numpy()
-    assert _rel2(got, want) <= (2.0 ** -18 if tokens * top_k <= 128 else 2.0 ** -10)
     for w in ws:
         w.free()
+    return y.numpy(), want
+
+
+@pytest.mark.parametrize("qg,qd,tokens,top_k,hidden,inter", [
+    ("q4_k", "q6_k", 1, 2, 256, 512), ("q5_k", "q5_k", 3, 2, 768, 256), ("iq4_xs", "q6_k", 2, 3, 512, 1280),
+    ("q8_0", "q8_0", 5, 1, 1280, 512), ("q6_k", "q4_k", 4, 2, 512, 768), ("iq4_xs", "iq4_xs", 1, 4, 4352, 256),
+    ("q5_k", "q6_k", 70, 2, 512, 512), ("q8_0", "iq4_xs", 66, 2, 256, 256)])
+@pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
+def test_moe_pairs_and_grouped(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, inter, x_dtype):
+    # up to 128 pairs: the f32 GEMVs (each product's sums below 2^-20, g and u through
+    # silu(g) * u and the down sums: four such errors, 2^-18).  More pairs: the grouped
+    # kernels, x and h in f16 (2^-11 each).  One id of the given ones is out of range and
+    # adds nothing.
+    _say("case: moe", qg, qd, tokens, top_k, hidden, inter, np.dtype(x_dtype).name)
+    got, want = _moe(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, inter, x_dtype)
+    assert _rel2(got, want) <= (2.0 ** -18 if tokens * top_k <= 128 else 2.0 ** -10)
+
+
+@pytest.mark.parametrize("q", ["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+def test_moe_pairs_lds_past_64k(gpu_ctx, oracle, q):
+    # x of gate and up, then of down, past the default LDS limit (16384 floats and their
+    # sums) after a short one in the same process: each kernel raises its own limit.
+    # The same bound as below 128 pairs above.
+    for hidden, inter in [(512, 512), (16384, 256), (256, 16384)]:
+        _say("case: moe lds", q, hidden, inter)
+        got, want = _moe(gpu_ctx, oracle, q, q, 2, 1, hidden, inter, np.float32)
+        assert _rel2(got, want) <= 2.0 ** -18
