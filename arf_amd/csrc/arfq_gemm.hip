@@ -339,7 +339,7 @@ static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 // direct: the direct-operand kernel where it takes the product
 static GemmPlan gemm_plan_of(const arfq_weight *w, int64_t m, int x_dtype, bool x16, bool direct) {
     GemmPlan p;
-    const int cus = w->ctx && w->ctx->cus > 0 ? w->ctx->cus : 256;
+    const int cus = w->cus;
     const bool kind2 = w->qtype == ARFQ_Q4_K || w->qtype == ARFQ_Q5_K;  // min term: x sums
     p.skinny = m <= 64 && w->k % 256 == 0;
     p.bm = m > 64 ? 128 : 64;

@@ -2028,7 +2028,7 @@ static hipError_t launch_gemv_t(const arfq_weight *w, int e, int m, const float 
 static int64_t q4k_gemv_grid(const arfq_weight *w) {
     const int nblk = (int)(w->k / 256);
     const int64_t steps = w->n * ((nblk + 3) / 4);
-    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    const int cus = w->cus;
     // two workgroups per CU; small problems get fewer (>= 2 steps per group)
     int64_t grid = std::min<int64_t>((int64_t)Q4K_GEMV_WG_PER_CU * cus,
                                      (steps + 2 * Q4K_GEMV_GROUPS - 1) / (2 * Q4K_GEMV_GROUPS));
@@ -2044,7 +2044,7 @@ static int64_t q4k_gemv_grid(const arfq_weight *w) {
 static int64_t gemv_grid(const arfq_weight *w, int groups) {
     const int nblk = (int)(w->k / 256);
     const int64_t steps = w->n * ((nblk + 3) / 4);
-    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    const int cus = w->cus;
     const int per_cu = w->k > 8192 ? 1 : 2;
     int64_t grid = std::min<int64_t>(per_cu * (int64_t)cus, (steps + 2 * groups - 1) / (2 * groups));
     grid = std::min<int64_t>(grid, w->n);
@@ -2102,13 +2102,13 @@ static size_t dot_f32_lds_rows(const arfq_weight *w, int64_t rows) {
 // waves per SIMD), while two workgroups' x and column sums fit the LDS.
 static int dot_f32_per_cu(const arfq_weight *w) {
     if (w->qtype != ARFQ_IQ4_XS || w->k > 8192) return 1;
-    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    const int cus = w->cus;
     return dot_f32_lds_rows(w, (w->n + 2 * cus - 1) / (2 * cus)) <= DOT_F32_LDS_MAX / 2 ? 2 : 1;
 }
 static int64_t dot_f32_grid(const arfq_weight *w) {
     const int nblk = (int)(w->k / 256);
     const int64_t steps = w->n * ((nblk + 3) / 4);
-    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    const int cus = w->cus;
     return std::max<int64_t>(1, std::min<int64_t>({(int64_t)dot_f32_per_cu(w) * cus, w->n,
                                                    (steps + 2 * Q6K_GEMV_GROUPS - 1) / (2 * Q6K_GEMV_GROUPS)}));
 }
@@ -2214,7 +2214,7 @@ static int q4k_f32_xr(const arfq_weight *w, int threads = Q4K_GEMV_THREADS) {
 // Small problems get fewer workgroups (>= 2 steps per 16-lane group).
 static int64_t q4k_f32s_grid(const arfq_weight *w) {
     const int64_t steps = w->n * ((w->k / 256 + 3) / 4);
-    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    const int cus = w->cus;
     int64_t grid = std::min<int64_t>(cus, (steps + 2 * (Q4K_F32_THREADS / 16) - 1) / (2 * (Q4K_F32_THREADS / 16)));
     grid = std::min<int64_t>(grid, w->n);
     return grid < 1 ? 1 : grid;
@@ -2308,7 +2308,7 @@ static int pairs_per_cu(int64_t P) { return P <= 8 ? 1 : 2; }
 // Workgroups per pair and weight, nz weights in the launch: about that many per CU over
 // all of them, >= 4 rows each.
 static int64_t pairs_grid(const arfq_weight *w, int64_t P, int nz) {
-    const int cus = w->ctx->cus > 0 ? w->ctx->cus : 256;
+    const int cus = w->cus;
     return std::max<int64_t>(1, std::min<int64_t>((pairs_per_cu(P) * (int64_t)cus + nz * P - 1) / (nz * P), w->n / 4));
 }
 static size_t dot_pairs_lds(const arfq_weight *w, int64_t g) { return dot_f32_lds_rows(w, (w->n + g - 1) / g); }

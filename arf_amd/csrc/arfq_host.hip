@@ -197,7 +197,8 @@ static int weight_create(arfq_ctx *ctx, int qtype, size_t nbytes, int64_t n_rows
     if (int rc = use_device(ctx)) return rc;
     arfq_weight *w = new (std::nothrow) arfq_weight();
     if (!w) return fail(ctx, ARFQ_E_NOMEM, "weight upload: host allocation");
-    w->ctx = ctx;
+    w->device = ctx->device;
+    w->cus = ctx->cus > 0 ? ctx->cus : 256;
     w->qtype = qtype;
     w->n = n_rows;
     w->k = k_cols;
@@ -309,7 +310,7 @@ int arfq_weight_upload(arfq_ctx *ctx, int qtype, const void *host_blocks, size_t
 
 int arfq_weight_free(arfq_weight *w) {
     if (!w) return ARFQ_E_INVALID;
-    if (w->ctx) (void)hipSetDevice(w->ctx->device);
+    (void)hipSetDevice(w->device);
     if (w->s0) (void)hipFree(w->s0);
     if (w->s1) (void)hipFree(w->s1);
     if (w->s2) (void)hipFree(w->s2);

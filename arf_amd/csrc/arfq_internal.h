@@ -33,7 +33,8 @@ struct arfq_ctx {
 };
 
 struct arfq_weight {
-    arfq_ctx *ctx = nullptr;
+    int device = 0;  // its GPU and that GPU's compute units (the context may go first)
+    int cus = 256;
     int qtype = 0;
     int64_t n = 0, k = 0;
     int experts = 1;

@@ -701,7 +701,7 @@ static unsigned moe_grid(const void *fn, int threads, size_t lds, std::atomic<in
             per_cu = 1;
         fit.store(per_cu, std::memory_order_relaxed);
     }
-    const int64_t cus = w->ctx && w->ctx->cus > 0 ? w->ctx->cus : 1;
+    const int64_t cus = w->cus;
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(max_items, per_cu * cus));
 }
 

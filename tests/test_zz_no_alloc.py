@@ -105,3 +105,18 @@ def test_noalloc_allocates_nothing():
         assert ctx.memory()[0] > 0  # arfq_matmul grew the context's scratch
     finally:
         ctx.close()
+
+
+def test_weight_outlives_its_context():
+    # a weight is freed after its context: the free goes to the weight's own GPU and
+    # leaves no error for the next call
+    from arf_amd import QType, synth
+    _say("case: weight outlives context")
+    n, k = 64, 256
+    for _ in range(8):
+        ctx = arf_amd.Context(0)
+        w = ctx.upload(QType.Q6_K, synth.weight("q6_k", n, k, seed=8), n, k)
+        ctx.close()
+        with arf_amd.Context(0) as other:
+            w.free()
+            other.upload(QType.Q6_K, synth.weight("q6_k", n, k, seed=9), n, k).free()
