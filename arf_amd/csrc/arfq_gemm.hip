@@ -444,6 +444,13 @@ GemmPlan gemm_plan(const arfq_weight *w, int64_t m, int x_dtype, bool x16, size_
     return p;
 }
 
+// one row group of 1 KiB per wave (32 weight rows) of each of the splits' column tiles, of
+// which there are at most two per CU when there is more than one split
+size_t plan_part_bytes(int cus) { return (size_t)2 * (cus > 0 ? cus : 256) * (sk_ct(1) / 32) * 1024; }
+bool plan_keeps_scratch(const arfq_weight *w, int64_t m, const GemmPlan &p) {
+    return p.fx && m <= 4 && (w->qtype == ARFQ_Q6_K || w->qtype == ARFQ_Q8_0);
+}
+
 template <class F, int TA, int PARTS, int GM = 0xFF, class XT = _Float16>
 static hipError_t launch_sk_t(const F &fmt, const arfq_weight *w, int64_t m, const XT *x,
                               const uint16_t *xs, const float *rs, int rss, float *y, float *part,

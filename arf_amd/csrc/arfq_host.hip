@@ -126,6 +126,10 @@ int arfq_ctx_create(int device, void *stream, arfq_ctx **out) {
         // flag words
         e = hipMalloc(&ctx->aux, ((size_t)arfq::STREAM_SINK_WORDS + arfq::UPLOAD_FLAG_WORDS) * sizeof(uint32_t));
     }
+    if (e == hipSuccess) {
+        ctx->part_bytes = arfq::plan_part_bytes(ctx->cus);
+        e = hipMalloc(&ctx->part, ctx->part_bytes);
+    }
     if (e == hipSuccess)
         e = hipMemsetAsync(ctx->aux, 0, ((size_t)arfq::STREAM_SINK_WORDS + arfq::UPLOAD_FLAG_WORDS) * sizeof(uint32_t),
                            ctx->stream);
@@ -145,6 +149,7 @@ int arfq_ctx_destroy(arfq_ctx *ctx) {
     if (ctx->stream && ctx->scratch) (void)hipFreeAsync(ctx->scratch, ctx->stream);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->staging) (void)hipFree(ctx->staging);
+    if (ctx->part) (void)hipFree(ctx->part);
     if (ctx->aux) (void)hipFree(ctx->aux);
     if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
     if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
@@ -358,6 +363,11 @@ static int ensure_scratch(arfq_ctx *ctx, size_t bytes) {
     return ARFQ_OK;
 }
 
+// Whether the plan's scratch is the context's fixed block.
+static bool scratch_in_part(const arfq_ctx *ctx, const arfq_weight *w, int64_t m, const arfq::GemmPlan &plan) {
+    return arfq::plan_keeps_scratch(w, m, plan) && plan.scratch_bytes <= ctx->part_bytes;
+}
+
 static int matmul_enqueue(arfq_ctx *ctx, const arfq_weight *w, int expert, int64_t m,
                           const void *x, int x_dtype, float *y) {
     hipError_t e;
@@ -368,8 +378,9 @@ static int matmul_enqueue(arfq_ctx *ctx, const arfq_weight *w, int expert, int64
         e = arfq::launch_gemv_f16(w, expert, x, y, ctx->stream);
     } else if (arfq::gemm_supports(w, m)) {
         const arfq::GemmPlan plan = arfq::gemm_plan(w, m, x_dtype, x16);
-        if (int rc = ensure_scratch(ctx, plan.scratch_bytes)) return rc;
-        e = arfq::launch_gemm(w, expert, m, x, x_dtype, y, ctx->scratch, plan, ctx->stream);
+        const bool part = scratch_in_part(ctx, w, m, plan);
+        if (int rc = ensure_scratch(ctx, part ? 0 : plan.scratch_bytes)) return rc;
+        e = arfq::launch_gemm(w, expert, m, x, x_dtype, y, part ? ctx->part : ctx->scratch, plan, ctx->stream);
     } else {
         return fail(ctx, ARFQ_E_UNSUPPORTED,
                     "matmul: no kernel for qtype " + std::to_string(w->qtype) + " at m=" +
@@ -400,14 +411,16 @@ int arfq_matmul_noalloc(arfq_ctx *ctx, const arfq_weight *w, int expert, int64_t
         e = arfq::launch_gemv_f16(w, expert, x, y, ctx->stream);
     } else if (arfq::gemm_supports(w, m)) {
         const arfq::GemmPlan plan = arfq::gemm_plan(w, m, x_dtype, x16, ARFQ_NOALLOC_SCRATCH_BYTES);
-        if (plan.scratch_bytes > ARFQ_NOALLOC_SCRATCH_BYTES)
+        const bool part = scratch_in_part(ctx, w, m, plan);
+        if (!part && plan.scratch_bytes > ARFQ_NOALLOC_SCRATCH_BYTES)
             return fail(ctx, ARFQ_E_UNSUPPORTED,
                         "matmul_noalloc: this product needs " + std::to_string(plan.scratch_bytes) +
                             " bytes of scratch, above the " + std::to_string(ARFQ_NOALLOC_SCRATCH_BYTES) +
                             "-byte limit (use arfq_matmul)");
         // every scratch byte a plan reads is written earlier in the same call
         // (x preparation, then the split-K partials before the launch that adds them)
-        e = arfq::launch_gemm(w, expert, m, x, x_dtype, y, ctx->noalloc_scratch, plan, ctx->stream);
+        e = arfq::launch_gemm(w, expert, m, x, x_dtype, y, part ? ctx->part : ctx->noalloc_scratch, plan,
+                              ctx->stream);
     } else {
         return fail(ctx, ARFQ_E_UNSUPPORTED,
                     "matmul_noalloc: no kernel for qtype " + std::to_string(w->qtype) + " at m=" +
@@ -660,10 +673,11 @@ int arfq_moe_ids_add(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight *
 
 // -------------------------------------------------------------------- FFN ----
 
-// Scratch bytes a matmul of w at m rows needs (GEMM plans; the GEMV needs none).
-static size_t matmul_scratch(const arfq_weight *w, int64_t m, bool x16) {
-    if (arfq::gemv_supports(w, m, x16)) return 0;
-    return arfq::gemm_supports(w, m) ? arfq::gemm_plan(w, m, ARFQ_F32, x16).scratch_bytes : 0;
+// Context scratch that a matmul of w at m rows needs (GEMM plans; the GEMV needs none).
+static size_t matmul_scratch(const arfq_ctx *ctx, const arfq_weight *w, int64_t m, bool x16) {
+    if (arfq::gemv_supports(w, m, x16) || !arfq::gemm_supports(w, m)) return 0;
+    const arfq::GemmPlan plan = arfq::gemm_plan(w, m, ARFQ_F32, x16);
+    return scratch_in_part(ctx, w, m, plan) ? 0 : plan.scratch_bytes;
 }
 
 int arfq_ffn_act(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight *up, const arfq_weight *down,
@@ -686,8 +700,8 @@ int arfq_ffn_act(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight *up, 
     // the activation applied as the down GEMV reads its x (Q4_K, m <= 4)
     const bool fused = arfq::gemv_glu_supports(down, m, x16);
     // the GEMM plans use the scratch from offset 0; g, u (and h) sit above the largest
-    size_t base = std::max({matmul_scratch(gate, m, x16), matmul_scratch(up, m, x16),
-                            fused ? (size_t)0 : matmul_scratch(down, m, x16)});
+    size_t base = std::max({matmul_scratch(ctx, gate, m, x16), matmul_scratch(ctx, up, m, x16),
+                            fused ? (size_t)0 : matmul_scratch(ctx, down, m, x16)});
     base = align256(base);
     const size_t gb = align256((size_t)m * inter * 4);
     if (int rc = ensure_scratch(ctx, base + (fused ? 2 : 3) * gb)) return rc;

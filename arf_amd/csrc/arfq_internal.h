@@ -22,6 +22,11 @@ struct arfq_ctx {
     // (stream-ordered allocations: grown without waiting for the stream)
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    // split-K partials of the products that plan_keeps_scratch names: allocated with
+    // the context and never moved, so that they neither allocate nor share scratch with
+    // another context, as the GEMVs that small products of their kind run
+    void *part = nullptr;
+    size_t part_bytes = 0;
     // staging of host uploads, reused across calls (at most UPLOAD_CHUNK bytes)
     void *staging = nullptr;
     size_t staging_bytes = 0;
@@ -150,6 +155,10 @@ struct GemmPlan {
 // limit: the scratch a caller with a fixed one has; a plan above it does not run there
 GemmPlan gemm_plan(const arfq_weight *w, int64_t m, int x_dtype, bool x16 = false, size_t limit = SIZE_MAX);
 bool gemm_supports(const arfq_weight *w, int64_t m);
+// Q6_K and Q8_0 at m = 2..4 (f32 x): the plan's scratch is arfq_ctx::part, of
+// plan_part_bytes, which holds it on every device
+bool plan_keeps_scratch(const arfq_weight *w, int64_t m, const GemmPlan &p);
+size_t plan_part_bytes(int cus);
 // y[m, n] = x[m, k] . W_e^T; `scratch` holds plan.scratch_bytes.
 hipError_t launch_gemm(const arfq_weight *w, int e, int64_t m, const void *x, int x_dtype,
                        float *y, void *scratch,

@@ -161,7 +161,10 @@ int arfq_matmul(arfq_ctx *ctx, const arfq_weight *w, int expert, int64_t m, cons
  * scratch (x preparation, split-K partials) from a fixed 32 MiB device array
  * per GPU instead of the context's growable buffer; a product that would need
  * more returns ARFQ_E_UNSUPPORTED (decode shapes, m <= 64 at k, n up to ~20K,
- * fit; the GEMVs need none).  Every call on a GPU shares that GPU's array:
+ * fit; the GEMVs need none, and Q6_K and Q8_0 at m = 2..4 keep their partials in
+ * a block that the context holds from its creation).  IQ4_XS above 64 rows at f32
+ * x runs the tile loop (arfq_matmul) where the prefill kernel's partials exceed
+ * the array.  Every call on a GPU shares that GPU's array:
  * calls that overlap on one GPU (two streams, two threads) race and must be
  * ordered by the caller.  No counterpart in the reference: for callers that
  * cannot allocate -- code under HIP graph capture, tight serving loops,
@@ -252,7 +255,8 @@ int arfq_stream_read(arfq_ctx *ctx, const void *src, size_t bytes, uint64_t *sta
  * in the reference (its adapter info comes from wgpu). */
 int arfq_ctx_device_info(arfq_ctx *ctx, int *cus, int *shader_clock_khz, int *wall_clock_khz);
 /* The device scratch the context holds (grown on demand by arfq_matmul,
- * arfq_moe* and arfq_ffn*; never by arfq_matmul_noalloc) and the device's free
+ * arfq_moe* and arfq_ffn*; never by arfq_matmul_noalloc; without the fixed 2 MiB
+ * that every context allocates) and the device's free
  * and total memory (hipMemGetInfo); any pointer may be NULL.  No counterpart
  * in the reference. */
 int arfq_ctx_memory(arfq_ctx *ctx, size_t *scratch_bytes, size_t *device_free, size_t *device_total);

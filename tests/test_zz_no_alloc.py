@@ -120,3 +120,34 @@ def test_weight_outlives_its_context():
         with arf_amd.Context(0) as other:
             w.free()
             other.upload(QType.Q6_K, synth.weight("q6_k", n, k, seed=9), n, k).free()
+
+
+@pytest.mark.parametrize("qtype,n,k", [("q6_k", 130, 16384), ("q6_k", 20000, 4096), ("q8_0", 5120, 8192)])
+@pytest.mark.parametrize("m", [2, 4])
+def test_small_m_keeps_no_shared_scratch(qtype, n, k, m):
+    # Q6_K and Q8_0 at 2..4 rows: neither entry point grows the context's scratch (as the
+    # GEMVs of small products), the outputs are the same bits, and calls of two contexts
+    # that overlap on their own streams do not meet in any scratch
+    from arf_amd import QType, synth
+    _say("case: small m scratch", qtype, n, k, m)
+    L = arf_amd.load_library()
+    ctxs = [arf_amd.Context(0) for _ in range(2)]
+    try:
+        calls = []
+        for i, ctx in enumerate(ctxs):
+            w = ctx.upload(QType[qtype.upper()], synth.weight(qtype, n, k, seed=90 + i), n, k)
+            x, y, z = ctx.to_device(synth.activations(m, k, seed=92 + i)), *(ctx.empty((m, n), np.float32) for _ in "yz")
+            ctx.matmul(w, x, m, y)
+            assert ctx.memory()[0] == 0
+            calls.append((ctx, w, x, z, y.numpy()))
+        for _ in range(20):
+            for ctx, w, x, z, _y in calls:
+                st = L.arfq_matmul_noalloc(ctx.handle, w.handle, 0, m, x.ptr, int(arf_amd.DType.F32), z.ptr)
+                assert st == arfq.ARFQ_OK, L.arfq_last_error(ctx.handle)
+        for ctx, w, x, z, y in calls:
+            assert ctx.memory()[0] == 0
+            assert np.array_equal(z.numpy().view(np.uint32), y.view(np.uint32))
+            w.free()
+    finally:
+        for ctx in ctxs:
+            ctx.close()
