@@ -177,7 +177,13 @@ __global__ __launch_bounds__(sk_nt(TA), TA == 4 ? 1 : 2) void gemm_sk(F fmt, con
     }
     if constexpr (PARTS == 3) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc[0][0][i] = (acc[0][0][i] + acc[0][0][i + 4]) + acc[0][0][i + 8];
+        for (int i = 0; i < 4; i++) {
+            if constexpr (FX && (GM & SK_SMALL))
+                acc[0][0][i] = fmaf(acc[0][0][i + 8], 1.f / (SK_WIDE * SK_WIDE),
+                                    fmaf(acc[0][0][i + 4], 1.f / SK_WIDE, acc[0][0][i]));
+            else
+                acc[0][0][i] = (acc[0][0][i] + acc[0][0][i + 4]) + acc[0][0][i + 8];
+        }
     }
     if (S == 1) {
 #pragma unroll
@@ -363,7 +369,8 @@ static GemmPlan gemm_plan_of(const arfq_weight *w, int64_t m, int x_dtype, bool 
     // half of the 32-row tile at m <= 16 (no extra MFMAs), a second tile at
     // m <= 32 and two more at m <= 64 (twice the MFMAs).  With x16
     // (ARFQ_OPT_GEMV_X16): one part, x rounded to f16.
-    // Q6_K and Q8_0 at m <= 4 have no 16-bit form to opt into and stay exact.
+    // Q6_K and Q8_0 at m <= 4 have no 16-bit form to opt into and keep the three parts
+    // (there held in units of their own: exact within 2^39 of the max, SK_SMALL).
     const bool exact4 = m <= 4 && (w->qtype == ARFQ_Q6_K || w->qtype == ARFQ_Q8_0);
     p.parts = p.skinny && x_dtype == ARFQ_F32 && (!x16 || exact4) ? (m <= 8 ? 3 : 2) : p.bd && bdx == 2 ? 2 : 1;
     // three parts (and their sub-block sums): formed by the skinny kernel as it
@@ -481,8 +488,8 @@ template <class F, int PARTS, class XT>
 static hipError_t launch_sk_m8(const F &fmt, const arfq_weight *w, int64_t m, const XT *x, const uint16_t *xs,
                                const float *rs, int rss, float *y, float *part, int S, hipStream_t s) {
     constexpr int GM = F::KIND < 3 ? 0xFF : PARTS == 3 ? 0x7 : 0x1;
-    if constexpr (std::is_base_of_v<SkQ6K, F> && PARTS == 3)
-        if (m <= 4) return launch_sk_t<F, 1, 3, GM | SK_OWN, XT>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
+    if constexpr (PARTS == 3 && (std::is_base_of_v<SkQ6K, F> || std::is_same_v<SkQ80, F>))
+        if (m <= 4) return launch_sk_t<F, 1, 3, GM | SK_SMALL, XT>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
     return launch_sk_t<F, 1, PARTS, GM, XT>(fmt, w, m, x, xs, rs, rss, y, part, S, s);
 }
 

@@ -435,8 +435,14 @@ struct SkRows {
     int64_t s;      // element offset (row * K / 16) of row min(tid >> 1, XR - 1)
 };
 
-// a bit of GM (Q6_K at m <= 4): an infinite x stays one, and KIND 4 sums each block apart
-constexpr int SK_OWN = 0x100;
+// A bit of GM: Q6_K and Q8_0 at f32 x and m <= 4, where f32 GEMVs take the smaller products
+// and took all.  The parts of x are held so that x within 2^39 of its row's largest is exact
+// and the rest off by at most 2^-63 of that (2^15 and 2^-39 with all parts in one unit; an
+// outlier that meets weights of 0 must not swamp the others), and Q6_K's KIND 4 sums each
+// block apart.  Q8_0 at m = 2..4 takes 1 % longer with it (17408 x 5120 27.9 -> 28.1 us at
+// m = 4), Q6_K no longer.
+constexpr int SK_SMALL = 0x100;
+constexpr float SK_WIDE = 4096.f;
 
 // LDS of the loop: XB buffers of the x block of XR rows (+ its sub-block sums)
 // and one weight slab [32][RB + 16] per wave and weight.
@@ -649,18 +655,21 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
     };
     auto xstore = [&](int to) {
         if constexpr (XP == 3) {
+            constexpr bool SMALL = (GM & SK_SMALL) != 0;
             half8 hp[3];
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const float u = ldexpf(__uint_as_float(xv[i >> 2][i & 3]), xsh);
                 hp[0][i] = (_Float16)u;
                 float r1 = u - (float)hp[0][i];  // exact
-                // an infinity is its own hi part, as the GEMVs of these formats multiply
-                // it (inf - inf would make every sum of the row NaN); Q6_K only at m <= 4,
-                // which had a GEMV: at m = 8 the compare took 28.6 -> 29.1 us
-                if constexpr (KIND == 3 ? F::OWN : (GM & SK_OWN) != 0) r1 = (float)hp[0][i] == u ? 0.f : r1;
+                // beside an infinite hi, mid and lo are any finite number (inf - inf would
+                // make every sum of the row NaN; |r1| <= 8 otherwise).  SK_SMALL: mid and
+                // lo are held 2^12 and 2^24 times up
+                if constexpr (SMALL || (KIND == 3 && F::OWN)) r1 = fmaxf(r1, -8.f);
+                if constexpr (SMALL) r1 *= SK_WIDE;
                 hp[1][i] = (_Float16)r1;
-                hp[2][i] = (_Float16)(r1 - (float)hp[1][i]);  // exact difference
+                const float r2 = r1 - (float)hp[1][i];  // exact
+                hp[2][i] = (_Float16)(SMALL ? r2 * SK_WIDE : r2);
             }
 #pragma unroll
             for (int q = 0; q < 3; q++)
@@ -789,7 +798,7 @@ __device__ __forceinline__ void skinny_loop(const F (&fmt)[NW], const int64_t (&
         // keep the scheduler from sinking the loads: they must be in flight
         // during this block, not issued at its end
         __builtin_amdgcn_sched_barrier(0);
-        sk_block<F, TA, TU, NW, GM, MERGE, PIN, XP == 3 && F::OWN && (KIND == 3 || (GM & SK_OWN)), XP != 3>(
+        sk_block<F, TA, TU, NW, GM, MERGE, PIN, XP == 3 && F::OWN && (KIND == 3 || (GM & SK_SMALL)), XP != 3>(
             slab, wb, [&](int t) { return xl + (xb * XR + 32 * t + lr) * SK_XLD; },
             [&](int t) { return sl + (xb * XR + 32 * t + lr) * 16; }, lr, h, acc, cb, cq);
 #pragma unroll

@@ -134,8 +134,9 @@ int arfq_weight_info(const arfq_weight *w, int *qtype, int64_t *n_rows, int64_t 
  *   - m <= 8 (Q4_K / Q5_K / IQ4_XS and larger Q6_K / Q8_0 products from m = 2): the
  *     skinny MFMA kernel with x as three f16 parts (hi + mid + lo) of x scaled
  *     per row (and per K range) by a power of two that puts the row's max |x|
- *     in [2^14, 2^15), so every x within 2^15 of that max is represented
- *     exactly; exact codes, f32 sums, the output scaled back.
+ *     in [2^14, 2^15), so every x within 2^15 of that max (2^39 for Q6_K and
+ *     Q8_0 at m <= 4, whose mid and lo parts have units of their own) is
+ *     represented exactly; exact codes, f32 sums, the output scaled back.
  *   - m = 9..64: the same with two parts (hi + lo, ~22 bits).
  *   - Above 64 rows: hi + lo of x scaled per row, in the prefill GEMM (twice
  *     the MFMAs of an f16 x).

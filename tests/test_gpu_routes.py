@@ -169,6 +169,30 @@ def test_moe_pairs_infinite_h(gpu_ctx, oracle, qd):
         w.free()
 
 
+@pytest.mark.parametrize("qtype,m,n,k,wide", [("q8_0", 2, 4200, 3840, False), ("q8_0", 4, 1024, 16384, False),
+                                              ("q6_k", 3, 130, 4352, True), ("q6_k", 4, 130, 4352, False),
+                                              ("q6_k", 2, 17, 16384, True)])
+def test_small_m_outlier_x(gpu_ctx, oracle, qtype, m, n, k, wide):
+    # an x 2^30 above its row's others that meets weights of 0 leaves their products as
+    # exact as f32 has them: the bound of test_small_m_q6_k_q8_0
+    _say("case: small m outlier", qtype, m, n, k, wide)
+    raw, x = synth.weight(qtype, n, k, seed=15), synth.activations(m, k, seed=16)
+    at = k - 600
+    if qtype == "q8_0":
+        raw.reshape(n, k // 32, 34)[:, at // 32, 2 + at % 32] = 0  # the code
+    else:
+        b = raw.reshape(n, k // 256, 210)
+        if wide:
+            b[:, :, 192:208] = np.random.default_rng(n).integers(0, 256, size=(n, k // 256, 16), dtype=np.uint8)
+        b[:, at // 256, 192 + at % 256 // 16] = 0  # the scale of its 16 elements
+    x[0, at], x[1, at] = 2.0 ** 30, -(2.0 ** 30)
+    w = gpu_ctx.upload(QType[qtype.upper()], raw, n, k)
+    y = gpu_ctx.empty((m, n), np.float32)
+    gpu_ctx.matmul(w, gpu_ctx.to_device(x), m, y)
+    assert _rel2(y.numpy(), _want(oracle, qtype, x, raw, n)) <= 2.0 ** -20
+    w.free()
+
+
 @pytest.mark.parametrize("qtype,n,k,wide", [("q8_0", 4200, 3840, False), ("q6_k", 130, 4352, True),
                                             ("q6_k", 130, 4352, False)])
 def test_small_m_infinite_x(gpu_ctx, oracle, qtype, n, k, wide):
