@@ -1442,7 +1442,9 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot(F fmt, const float 
 // weight (gguf.rs:2120-2123) times f32 x, factorised.
 namespace {
 
-// (returns whether the sum of the thread's 16 elements, times a code, may not be finite)
+// (returns whether the sum of the thread's 16 elements, times a code, may not be finite;
+// INFX: the kernel keeps an infinite x)
+template <bool INFX>
 __device__ __forceinline__ bool xf16_process(const XqRound &r, int items, int base, float4 *xf,
                                              float *s16, float *xe) {
     const int it = base + (int)threadIdx.x;
@@ -1454,7 +1456,7 @@ __device__ __forceinline__ bool xf16_process(const XqRound &r, int items, int ba
     sum += quad_perm<QP_XOR1>(sum);  // 16 elements (items 2i, 2i + 1)
     amax = fmaxf(amax, quad_perm<QP_XOR2>(amax));
     // (beside an infinity, whose exponent reads as 0, the finite elements must not overflow)
-    const int ex = amax == INFINITY ? 128 : (amax > 0.f) ? __builtin_amdgcn_frexp_expf(amax) : 0;
+    const int ex = INFX && amax == INFINITY ? 128 : (amax > 0.f) ? __builtin_amdgcn_frexp_expf(amax) : 0;
     const int sh = min(24, 100 - ex);
     if (it < items) {
         xf[2 * it] = make_float4(ldexpf(v0.x, sh), ldexpf(v0.y, sh), ldexpf(v0.z, sh), ldexpf(v0.w, sh));
@@ -1508,23 +1510,26 @@ __device__ __forceinline__ float codes16_sdot(const uint32_t cw[4], const float 
 // narrow window of the weight stream at a time), and x is scaled into LDS
 // before the first weight load is issued (every weight request in flight
 // delays the x requests); as the Q4_K f32 GEMV (gemv_q4k_f32_body).
-// Formats with a BIAS: an x whose sum over some quadrant is not finite (the bytes less
-// BIAS * sum(x) would be inf - inf for every code) has its rows done again at the end
-// with the signed codes.  IQ4_XS takes those for every f16 x (SG: 16.1 -> 18.1 us at
-// 17408 x 5120, but error against 64 bits 1.04e-7 -> 7.5e-8 at 4096 x 1024; the skinny
-// kernel, without a bias to cancel, has 8.2e-8.  At f32 x the bytes' 2.0e-7 would be
-// 1.0e-7, for 11 % more time, 6 % for Q6_K; a branch on x in the loop took 28
-// registers).
+// Formats with a BIAS, REDO (an f16 row and the MoE pairs, which the MFMA kernels ran on
+// signed codes): an x whose sum over some quadrant is not finite (the bytes less BIAS *
+// sum(x) would be inf - inf for every code) has its rows done again at the end with the
+// signed codes.  One f32 row is without it (NaN): beside the loop it took IQ4_XS 5120 x
+// 5120 9.88 -> 10.07 us, Q6_K 3000 x 9216 9.15 -> 9.31.  IQ4_XS takes the signed codes
+// for every f16 row (SG: 16.1 -> 18.1 us at 17408 x 5120, but error against 64 bits
+// 1.04e-7 -> 7.5e-8 at 4096 x 1024; the skinny kernel, without a bias to cancel, has
+// 8.2e-8.  At f32 x the bytes' 2.0e-7 would be 1.0e-7, for 11 % more time, 6 % for Q6_K; a
+// branch on x in the loop took 28 registers).
 template <class F, int XR, class XSRC>
 __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc, float *__restrict__ y, int n,
                                                   int nblk) {
     constexpr bool SG = F::BIAS == 128 && std::is_same_v<XSRC, XsF16>;
+    constexpr bool REDO = F::BIAS != 0 && !SG && !std::is_same_v<XSRC, XsF32>;
     constexpr int C = Q6K_GEMV_CHUNK, PF = F::PF;
     static_assert(PF % C == 0, "claims must sit at fixed slots of the unrolled loop");
     extern __shared__ uint4 smem4[];
     __shared__ int cnt[64];             // chunk counters per column (spr <= 64)
     __shared__ unsigned long long exm;  // columns seen exhausted
-    __shared__ int redo;                // some sum(x) is not finite
+    __shared__ int redo;                // some sum(x) is not finite (REDO)
     const int k = nblk * 256;
     float *xfl = reinterpret_cast<float *>(smem4);  // [k], scaled
     float *s16 = xfl + k;                           // [k / 16]
@@ -1611,7 +1616,10 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
 
     // counters start past the chunks the groups begin on
     for (int cc = tid; cc < spr; cc += Q6K_GEMV_THREADS) cnt[cc] = (Q6K_GEMV_GROUPS - cc + spr - 1) / spr;
-    if (tid == 0) exm = 0, redo = 0;
+    if (tid == 0) {
+        exm = 0;
+        if constexpr (REDO) redo = 0;
+    }
     // x loads, x scaled into LDS, the barrier (which orders LDS only), then the
     // first weight loads
     const int xitems = k / 8;
@@ -1622,11 +1630,12 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
     bool odd = false;
 #pragma unroll
     for (int r = 0; r < XR; r++)
-        odd |= xf16_process(xr[r], xitems, r * Q6K_GEMV_THREADS, reinterpret_cast<float4 *>(xfl), s16, xe);
+        odd |= xf16_process<REDO || SG || F::SIGNED>(xr[r], xitems, r * Q6K_GEMV_THREADS, reinterpret_cast<float4 *>(xfl), s16, xe);
     for (int base = XR * Q6K_GEMV_THREADS; base < xitems; base += Q6K_GEMV_THREADS)
-        odd |= xf16_process(xsrc.load(xitems, base), xitems, base, reinterpret_cast<float4 *>(xfl), s16, xe);
+        odd |= xf16_process<REDO || SG || F::SIGNED>(xsrc.load(xitems, base), xitems, base, reinterpret_cast<float4 *>(xfl), s16, xe);
     lds_barrier();
-    if (F::BIAS != 0 && !SG && odd) redo = 1;  // read past the next barrier
+    if constexpr (REDO)
+        if (odd) redo = 1;  // read past the next barrier
 #pragma unroll
     for (int u = 0; u < PF; u++) issue(u, u < C);
 
@@ -1692,14 +1701,15 @@ __device__ __forceinline__ void gemv_dot_f32_body(const F &fmt, const XSRC &xsrc
     }
     lds_barrier();
 
-    const bool again = F::BIAS != 0 && !SG && redo;  // (read with the sums: no wait of its own)
+    bool again = false;
+    if constexpr (REDO) again = redo;
     for (int t = tid; t < R; t += Q6K_GEMV_THREADS) {
         const float *pr = part + (size_t)t * spr;
         float v = 0.f;
         for (int cc = 0; cc < spr; cc++) v += pr[cc];
         if (__builtin_expect(!again, 1)) y[r0 + t * G] = v;
     }
-    if constexpr (F::BIAS != 0 && !SG) {
+    if constexpr (REDO) {
         if (__builtin_expect(again, 0)) {  // a 16-lane group per row
             for (int row = grp; row < R; row += Q6K_GEMV_GROUPS) {
                 float v = 0.f;

@@ -125,13 +125,14 @@ def test_m1_q8_0_infinite_x(gpu_ctx, oracle):
     w.free()
 
 
-@pytest.mark.parametrize("qtype,n,k", [("q6_k", 130, 256), ("q6_k", 700, 4352), ("iq4_xs", 1030, 1792),
-                                       ("iq4_xs", 3, 8448), ("q8_0", 13000, 1280)])
-@pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("qtype,n,k,x_dtype", [
+    ("q6_k", 130, 256, np.float16), ("q6_k", 700, 4352, np.float16), ("iq4_xs", 1030, 1792, np.float16),
+    ("iq4_xs", 3, 8448, np.float16), ("q8_0", 13000, 1280, np.float16), ("q8_0", 13000, 1280, np.float32)])
 @pytest.mark.parametrize("at", [0, -3])
 def test_m1_infinite_x(gpu_ctx, oracle, qtype, n, k, x_dtype, at):
-    # +-inf by the sign of its weight, NaN (0 * inf) where that is 0, in one x row of f32 or
-    # f16: the first block, or a last column of one or three blocks
+    # +-inf by the sign of its weight, NaN (0 * inf) where that is 0, in one x row (f16; f32
+    # for Q8_0, whose f32 GEMVs all multiply signed codes): the first block, or a last
+    # column of one or three blocks
     _say("case: m1 inf", qtype, n, k, np.dtype(x_dtype).name, at)
     raw, x = synth.weight(qtype, n, k, seed=21), synth.activations(1, k, seed=22).astype(x_dtype)
     x[0, at] = -np.inf
