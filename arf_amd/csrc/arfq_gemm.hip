@@ -231,7 +231,10 @@ __global__ __launch_bounds__(sk_nt(TA), TA == 4 ? 1 : 2) void gemm_sk(F fmt, con
 // column tile * ct + 32 wave + lane % 32 (row group gi = 4 t + g).  All S loads
 // are in flight at once: straight-line code, the loads of splits past S reading
 // past the end of the buffer, which returns 0 and moves no data (adding that 0
-// changes nothing but a -0 sum into +0).
+// changes nothing but a -0 sum into +0).  PAIRS (SK_SMALL): added in pairs, which keeps Q8_0
+// at m = 2..4 no further from 64 bits than the f32 GEMV (9216 -> 3000: 1.09e-7 in one chain,
+// 9.5e-8 in pairs, the GEMV 1.03e-7).
+template <bool PAIRS>
 __global__ __launch_bounds__(256) void sk_reduce_kernel(const float *__restrict__ part, float *__restrict__ y,
                                                         int S, int nt, int nw, int GT, int ct, int M, int N) {
     const int64_t units = (int64_t)nt * nw * GT;  // float4 columns of one split, / 64
@@ -250,11 +253,21 @@ __global__ __launch_bounds__(256) void sk_reduce_kernel(const float *__restrict_
                                                               (uint32_t)(j >= S) << 31, 0, 0);
     float r[4];
 #pragma unroll
-    for (int c = 0; c < 4; c++) r[c] = __uint_as_float(d[0][c]);
+    for (int c = 0; c < 4; c++) {
+        float v[16];
 #pragma unroll
-    for (int j = 1; j < 16; j++)
+        for (int j = 0; j < 16; j++) v[j] = __uint_as_float(d[j][c]);
+        if constexpr (PAIRS) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) r[c] += __uint_as_float(d[j][c]);
+            for (int o = 1; o < 16; o *= 2)
+#pragma unroll
+                for (int j = 0; j + o < 16; j += 2 * o) v[j] += v[j + o];
+        } else {
+#pragma unroll
+            for (int j = 1; j < 16; j++) v[0] += v[j];
+        }
+        r[c] = v[0];
+    }
     const int row = 32 * (gi >> 2) + 8 * (gi & 3) + 4 * (lane >> 5);
     const int n = tile * ct + 32 * wave + (lane & 31);
 #pragma unroll
@@ -475,7 +488,7 @@ static hipError_t launch_sk_t(const F &fmt, const arfq_weight *w, int64_t m, con
     if (S > 1) {
         const int gt = (int)((m + 7) / 8);
         const int64_t threads = (int64_t)nt * (NT / 64) * gt * 64;
-        sk_reduce_kernel<<<(unsigned)((threads + 255) / 256), 256, 0, s>>>(part, y, S, nt, NT / 64, gt, CT, (int)m,
+        sk_reduce_kernel<(GM & SK_SMALL) != 0><<<(unsigned)((threads + 255) / 256), 256, 0, s>>>(part, y, S, nt, NT / 64, gt, CT, (int)m,
                                                                            (int)w->n);
         return hipGetLastError();
     }

@@ -269,3 +269,38 @@ def test_moe_pairs_lds_past_64k(gpu_ctx, oracle, q):
         _say("case: moe lds", q, hidden, inter)
         got, want = _moe(gpu_ctx, oracle, q, q, 2, 1, hidden, inter, np.float32)
         assert _rel2(got, want) <= 2.0 ** -18
+
+
+@pytest.mark.parametrize("qtype", ["q4_k", "q5_k", "q6_k", "iq4_xs", "q8_0"])
+@pytest.mark.parametrize("n,k", [(4096, 1024), (3000, 5120)])
+def test_f16_row_no_further_off_than_the_mfma_kernel(gpu_ctx, oracle, qtype, n, k):
+    # the f32 GEMVs that take one f16 row are no further from 64 bits than the skinny MFMA
+    # kernel, which takes the row beside a second one.  Over n outputs the two errors'
+    # ratio is known to a few parts in sqrt(n)
+    _say("case: f16 row error", qtype, n, k)
+    raw = synth.weight(qtype, n, k, seed=41)
+    x = np.repeat(synth.activations(1, k, seed=42).astype(np.float16), 2, axis=0)
+    w = gpu_ctx.upload(QType[qtype.upper()], raw, n, k)
+    y1, y2 = gpu_ctx.empty((1, n), np.float32), gpu_ctx.empty((2, n), np.float32)
+    gpu_ctx.matmul(w, gpu_ctx.to_device(x[:1]), 1, y1)
+    gpu_ctx.matmul(w, gpu_ctx.to_device(x), 2, y2)
+    want = _want(oracle, qtype, x[:1], raw, n)
+    assert _rel2(y1.numpy(), want) <= (1 + 4 / np.sqrt(n)) * _rel2(y2.numpy()[:1], want)
+    w.free()
+
+
+@pytest.mark.parametrize("m,n,k,wave", [(1, 1500, 30720, 1.16e-7), (3, 3000, 9216, 1.01e-7), (4, 1100, 30720, 1.19e-7)])
+def test_q8_0_no_further_off_than_the_one_wave_gemv(gpu_ctx, oracle, m, n, k, wave):
+    # the dot kernel at m = 1 and the skinny kernel at m = 2..4 add their columns and splits
+    # so that a long row is no further from 64 bits than in gemv_q80w, which took these
+    # products: `wave` is the lowest it measured over four such inputs (1.16 .. 1.23e-7,
+    # 1.01 .. 1.05e-7, 1.19 .. 1.20e-7)
+    _say("case: q8_0 long rows", m, n, k)
+    raw, x = synth.weight("q8_0", n, k, seed=0), synth.activations(m, k, seed=50)
+    w = gpu_ctx.upload(QType.Q8_0, raw, n, k)
+    y = gpu_ctx.empty((m, n), np.float32)
+    gpu_ctx.matmul(w, gpu_ctx.to_device(x), m, y)
+    b = raw.reshape(n, k // 32, 34)  # the product of d and q in 64 bits, as the kernels have it
+    wt = (b[:, :, :2].copy().view(np.float16).astype(np.float64) * b[:, :, 2:].view(np.int8)).reshape(n, k)
+    assert _rel2(y.numpy(), x.astype(np.float64) @ wt.T) <= wave
+    w.free()
