@@ -2528,7 +2528,7 @@ bool gemv_f16_supports(const arfq_weight *w, int64_t m) {
     if (m != 1) return false;
     switch (w->qtype) {
     case ARFQ_Q4_K: return q4k_f32s_ok(w);
-    case ARFQ_Q8_0: return w->k % 256 == 0;
+    case ARFQ_Q8_0: return gemm_supports(w, m);  // (k a multiple of 64: others take no f16 x)
     default: return dot_f32_ok(w);
     }
 }

@@ -129,7 +129,7 @@ int arfq_weight_info(const arfq_weight *w, int *qtype, int64_t *n_rows, int64_t 
  *   - m = 1: f32 x times the exact weights in f32 (Q4_K, Q5_K, IQ4_XS and Q6_K
  *     while x fits the kernels' LDS: k up to about 37K for Q4_K and 38K for the
  *     others; longer x takes the m <= 8 path below).
- *     An f16 x of one row takes the same kernels (Q8_0: k a multiple of 256).
+ *     An f16 x of one row takes the same kernels.
  *   - m <= 4: Q6_K and Q8_0 GEMVs in f32 for small products.
  *   - m <= 8 (Q4_K / Q5_K / IQ4_XS and larger Q6_K / Q8_0 products from m = 2): the
  *     skinny MFMA kernel with x as three f16 parts (hi + mid + lo) of x scaled
