@@ -282,7 +282,7 @@ def test_next_formats_skinny_and_prefill(gpu_ctx, oracle, qtype, m, n, k, x16):
     # Q5_K / IQ4_XS beyond the decode GEMV: the skinny MFMA kernel (m <= 64) and the
     # prefill above 64 rows; f16 x (the x16 cases) is what the oracle sees.  Exact
     # weights with x in f16 parts hold 2e-5: Q5_K everywhere at f32 x, IQ4_XS on the skinny
-    # kernel; the IQ4_XS prefill at f32 x runs the tile loop with weights rounded to f16
+    # kernel; the IQ4_XS prefill rounds (ls - 32) * kv to f16 where it passes 2048
     _say("case: next-format skinny", qtype, m, n, k, "f16" if x16 else "f32")
     dt = np.float16 if x16 else np.float32
     got, raw, x = _matmul(gpu_ctx, qtype, n, k, m, seed=11 * m + n, x_dtype=dt)
@@ -296,7 +296,7 @@ def test_next_formats_skinny_and_prefill(gpu_ctx, oracle, qtype, m, n, k, x16):
                                    (130, 64), (8, 62), (64, 62)])
 def test_q6_k_full_range_scales(gpu_ctx, oracle, m, lim):
     # quantizers put each block's largest sub-block scale near +-127, where sc * (q - 32)
-    # passes 2048 and would round in f16; the skinny kernel (m = 5..64) multiplies the exact
+    # passes 2048 and would round in f16; the skinny kernel (m = 8, 64) multiplies the exact
     # codes q - 32 and scales each sub-block's product by d * sc in f32, the prefill GEMM
     # (m = 130) holds sc * (q - 32) as f16 hi + lo operands (exact) against x as f16
     # hi + lo.  The synthetic blocks keep scales in [-32, 31], so this test draws them from
@@ -351,9 +351,10 @@ def test_vocab_wide_lm_head_gemv(gpu_ctx, oracle, qtype):
 # ---- f32 x over the batched decode range ----
 # m = 2..8 multiply f32 x in f32 terms: Q4_K / Q5_K / IQ4_XS on the skinny MFMA kernel
 # with x as three f16 parts (hi + mid + lo, which represent every f32 value within 2^15 of
-# its row's max |x| exactly; the exact codes times each part, f32 sums), Q6_K on the f32
-# GEMV at m <= 4, Q8_0 on its f32 GEMV at m <= 4.  m = 9..64: the skinny kernel with x as
-# f16 hi + lo (~22 bits).  Held to 2e-5 against the oracle.
+# its row's max |x| exactly; the exact codes times each part, f32 sums), Q6_K and Q8_0 at
+# m <= 4 on their f32 GEMVs or, larger products, on the same kernel (exact within 2^39 of
+# the max).  m = 9..64: the skinny kernel with x as f16 hi + lo (~22 bits).  Held to 2e-5
+# against the oracle.
 SMALL_M_TOL = 2e-5
 
 

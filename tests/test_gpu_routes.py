@@ -247,7 +247,7 @@ def _moe(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, inter, x_dtype):
 @pytest.mark.parametrize("qg,qd,tokens,top_k,hidden,inter", [
     ("q4_k", "q6_k", 1, 2, 256, 512), ("q5_k", "q5_k", 3, 2, 768, 256), ("iq4_xs", "q6_k", 2, 3, 512, 1280),
     ("q8_0", "q8_0", 5, 1, 1280, 512), ("q6_k", "q4_k", 4, 2, 512, 768), ("iq4_xs", "iq4_xs", 1, 4, 4352, 256),
-    ("q5_k", "q6_k", 70, 2, 512, 512), ("q8_0", "iq4_xs", 66, 2, 256, 256)])
+    ("q5_k", "q6_k", 70, 2, 512, 512), ("q8_0", "iq4_xs", 66, 2, 256, 256), ("q6_k", "q6_k", 70, 2, 256, 2048)])
 @pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
 def test_moe_pairs_and_grouped(gpu_ctx, oracle, qg, qd, tokens, top_k, hidden, inter, x_dtype):
     # up to 128 pairs: the f32 GEMVs (each product's sums below 2^-20, g and u through
