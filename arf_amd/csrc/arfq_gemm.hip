@@ -252,21 +252,27 @@ __global__ __launch_bounds__(256) void sk_reduce_kernel(const float *__restrict_
         d[j] = __builtin_amdgcn_raw_buffer_load_b128(prs, ((uint32_t)j * split_bytes + (uint32_t)q * 16u) |
                                                               (uint32_t)(j >= S) << 31, 0, 0);
     float r[4];
+    if constexpr (PAIRS) {
+        float v[16][4];
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-        float v[16];
+        for (int j = 0; j < 16; j++)
 #pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = __uint_as_float(d[j][c]);
-        if constexpr (PAIRS) {
+            for (int c = 0; c < 4; c++) v[j][c] = __uint_as_float(d[j][c]);
 #pragma unroll
-            for (int o = 1; o < 16; o *= 2)
+        for (int o = 1; o < 16; o *= 2)
 #pragma unroll
-                for (int j = 0; j + o < 16; j += 2 * o) v[j] += v[j + o];
-        } else {
+            for (int j = 0; j + o < 16; j += 2 * o)
 #pragma unroll
-            for (int j = 1; j < 16; j++) v[0] += v[j];
-        }
-        r[c] = v[0];
+                for (int c = 0; c < 4; c++) v[j][c] += v[j + o][c];
+#pragma unroll
+        for (int c = 0; c < 4; c++) r[c] = v[0][c];
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; c++) r[c] = __uint_as_float(d[0][c]);
+#pragma unroll
+        for (int j = 1; j < 16; j++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) r[c] += __uint_as_float(d[j][c]);
     }
     const int row = 32 * (gi >> 2) + 8 * (gi & 3) + 4 * (lane >> 5);
     const int n = tile * ct + 32 * wave + (lane & 31);

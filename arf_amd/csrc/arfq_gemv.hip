@@ -965,9 +965,10 @@ __device__ __forceinline__ int q6k_subdot(const uint32_t *cw, const u32x4 lo, co
 //
 // Q6_K: lane c = chunk c of the repacked block (16 bytes each of ql_a, ql_b and qh,
 // see q6k_off); q = ql nibble | qh bits << 4 (0..63); weight (d * sc) * (q - 32).
-// A load takes part of each 64-byte sector, so the loads are cached: non-temporal,
-// the sectors were fetched again for each of the three (5120 -> 151936 142.6 -> 105.7
-// us, 17408 -> 5120 20.4 -> 16.7).  Each sector read whole by one load (the block as
+// A load takes part of each cache line, so the loads are cached: non-temporal, each of
+// the three asked the L2 for the line again (17408 -> 5120: 1.78 M requests against
+// 0.73 M, the bytes from memory the same; 5120 -> 151936 142.6 -> 106.6 us, 17408 -> 5120
+// over rotating copies 20.7 -> 17.7).  Each sector read whole by one load (the block as
 // three planes) without the cache: 114 and 17.7 us.
 struct DotQ6K {
     const uint8_t *qb, *scb, *db;
@@ -1053,7 +1054,7 @@ struct DotQ6K {
 // 2 p + 1 (high), the fifth bits in bits 2 p and 2 p + 1 of qh[l0 ..].  Quadrant
 // t = sub-block 2 p + t % 2 of load t / 2.  (As 32 contiguous bytes per lane, a load
 // took 16 of every 32 bytes: 5120 -> 17408 19.0 -> 18.2 us; cached, as Q6_K's, since a
-// block's 160 bytes share 64-byte sectors with its neighbours': 16.3.)  Each lane loads a
+// block's 160 bytes share cache lines with its neighbours': 16.2, over rotating copies 17.0.)  Each lane loads a
 // quarter of qh (bytes 8c .. 8c + 7) and header dword c; expand() shares them over
 // the quad by DPP.  q = nibble | bit << 4 (0..31); weight (d * sc) * q - dmin * m
 // (crates/arf-core/src/model/gguf.rs:2053-2090).
@@ -1782,7 +1783,7 @@ __global__ __launch_bounds__(Q6K_GEMV_THREADS) void gemv_dot_pairs(F f0, F f1, X
 // Reference arithmetic: matmul_nt_q8_0 (crates/arf-ml/src/matmul.rs:174-204).
 // two waves per workgroup (twice as many workgroups as four): C1 3.91 -> 3.73 us
 // per launch; one row per wave or four rows per wave measured 4.5-4.7 us.  The loads
-// are cached: a lane's two take 16 bytes each of the same 64-byte sectors
+// are cached: a lane's two take 16 bytes each of the same cache lines
 // (non-temporal, 8192 x 1024 5.07 against 4.67 us).
 constexpr int Q80_WAVES = 2, Q80_ROWS = 2;
 template <int MX, class XT>
@@ -1992,8 +1993,8 @@ static bool q4k_x16_ok(const arfq_weight *w, int64_t m) {
 // 18.7; 2048 x 2048: 8.2 against 9.6).  Q8_0 from ~30M products on (m = 4,
 // 4096 x 4096: 19.1 -> 10.3; m = 3, 17408 -> 5120: 73 -> 26; m = 3, 4096 x 2048:
 // 8.5 against 9.9), not for the few rows that leave its waves short (1000 x
-// 18432: 14.6 against 15.6).  Error against 64 bits: 1.7e-7 -> 1.2e-7 (Q6_K),
-// unchanged at 1e-7 (Q8_0).
+// 18432: 14.6 against 15.6).  Error against 64 bits: 1.7e-7 -> 1.0e-7 (Q6_K),
+// 1.0e-7 -> 9.6e-8 (Q8_0).
 static bool skinny_m2_4(const arfq_weight *w, int64_t m) {
     if (m < 2 || w->k % 256 != 0 || w->n > INT32_MAX / 2 || w->k > INT32_MAX / 2) return false;
     const bool much = w->n * w->k >= 30000000 / m;

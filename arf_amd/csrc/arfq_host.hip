@@ -503,6 +503,7 @@ static int check_moe(arfq_ctx *ctx, const arfq_weight *gate, const arfq_weight *
 // 413 / 119.  Q4_K throughout always takes them: f32 arithmetic is what it has had.
 static bool moe_pairs_pay(const arfq_weight *gate, const arfq_weight *down, int64_t P) {
     if (gate->qtype == ARFQ_Q4_K && down->qtype == ARFQ_Q4_K) return true;
+    // (up is of gate's format and shape, down's shape holds as many weights: check_moe)
     const double E = gate->experts, w = (double)gate->n * gate->k * 1e-6;  // million weights
     auto mb = [&](const arfq_weight *t) { return w * arfq::block_bytes_of(t->qtype) / arfq::qk_of(t->qtype); };
     auto rate = [](const arfq_weight *t) { return t->qtype == ARFQ_IQ4_XS ? 3.3 : 5.8; };

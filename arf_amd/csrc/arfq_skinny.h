@@ -439,8 +439,8 @@ struct SkRows {
 // and took all.  The parts of x are held so that x within 2^39 of its row's largest is exact
 // and the rest off by at most 2^-63 of that (2^15 and 2^-39 with all parts in one unit; an
 // outlier that meets weights of 0 must not swamp the others), and Q6_K's KIND 4 sums each
-// block apart.  Q8_0 at m = 2..4 takes 1 % longer with it (17408 x 5120 27.9 -> 28.1 us at
-// m = 4), Q6_K no longer.
+// block apart.  Q8_0 at m = 2..4 takes 1 - 2 % longer with it (17408 x 5120 28.0 -> 28.4 us
+// at m = 4), Q6_K no longer.
 constexpr int SK_SMALL = 0x100;
 constexpr float SK_WIDE = 4096.f;
 

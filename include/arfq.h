@@ -91,7 +91,8 @@ int arfq_ctx_sync(arfq_ctx *ctx);
  *   exact integer dots; faster, max relative error ~1e-4 of the output's rms.
  *   Only where those kernels' LDS fits 64 KiB: longer x keeps the default
  *   path.  The skinny MFMA kernel and the prefill GEMM (below) then take an
- *   f32 x as one f16 part (11 bits) instead of two or three.
+ *   f32 x as one f16 part (11 bits) instead of two or three, except for Q6_K and
+ *   Q8_0 at m <= 4, which keep their three.
  *   By default every GEMV multiplies f32 x by the exact weights in f32,
  *   as the reference GEMVs do
  *   (crates/arf-gpu/src/shaders/metal/matmul_vec_q4ks_msl.metal:46-165,
@@ -144,7 +145,8 @@ int arfq_weight_info(const arfq_weight *w, int *qtype, int64_t *n_rows, int64_t 
  * and Q8_0 (Q6_K scales beyond +-64 and Q8_0's d * q as two f16 operands
  * above 64 rows), except in the tile loop that takes the shapes the direct
  * prefill kernel does not (Q8_0 with k not a multiple of 256, streams past
- * 2 GiB): there the dequant is rounded once to f16.  IQ4_XS weights are exact
+ * 2 GiB, IQ4_XS at f32 x whose partials exceed arfq_matmul_noalloc's array):
+ * there the dequant is rounded once to f16.  IQ4_XS weights are exact
  * up to 64 rows; above, (ls - 32) * kv is rounded to f16 where it passes 2048.
  * Replaces add_matmul_m / add_matmul
  * (crates/arf-gpu/src/gpu/dispatch.rs:169-202, Q4KS arms :517-630) and the
